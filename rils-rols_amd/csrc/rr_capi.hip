@@ -1171,20 +1171,36 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
   // first ne positions (more than TS_MAX_COLS columns) take the
   // step-synchronous QR: per step s the positions taking part (step_pos[s]:
   // those with more than s columns, a prefix) and their chunk work items
-  // (step_items[s]).  The rest take the chunked QR in three column buckets:
+  // (step_items[s]).  The rest take the chunked QR in column buckets:
   // positions ts_pos[i] .. ts_pos[i+1]-1 and chunk work items ts_it[i] ..
-  // ts_it[i+1]-1 have TS_NC[i] columns with y (positions and items relative to
-  // the chunk's first).
+  // ts_it[i+1]-1 are bucket i's (positions and items relative to the chunk's
+  // first).
   struct Chunk64 {
     int c0, c1, maxk, p0, npair, nitem, per, sitem, sper, ne, depth;
-    int ts_pos[4], ts_it[4];
+    int ts_pos[rr::TS_BUCKETS + 1], ts_it[rr::TS_BUCKETS + 1];
     int ts_maxch;       // the most chunk work items of a chunked-QR position
-    int64_t ts_lw[4];   // the buckets' work-item descriptors: first word, and the words in all
     std::vector<int32_t> step_pos, step_items;
   };
-  static constexpr int TS_NC[3] = {10, 5, 3};
   // a chunked-QR position has as many chunk work items as scoring ones
   static_assert(rr::TS_ROWS == rr::EVAL_CHUNK_ROWS, "chunked QR and scoring share the chunk numbering");
+  // the chunked QR's work lists (rr::TsList) of a launch chunk, one after the
+  // other in d_tslist: its words, and where they are
+  auto ts_list_words = [](const Chunk64& ch) -> int64_t {
+    const int64_t mc = ch.c1 - ch.c0;
+    return 2 * rr::TS_BUCKETS + 2 * mc + (ch.sper > 0 ? 0 : 2 * (int64_t)ch.sitem);
+  };
+  auto ts_list = [&](const Chunk64& ch) {
+    rr::TsList t{};
+    const int64_t mc = ch.c1 - ch.c0;
+    t.cnt = (int32_t*)ctx->d_tslist.p;
+    t.live = t.cnt + 2 * rr::TS_BUCKETS;
+    t.base = t.live + mc;
+    t.items = t.base + mc;
+    for (int i = 0; i <= rr::TS_BUCKETS; ++i) t.pos0[i] = ch.ts_pos[i];
+    for (int i = 0; i < rr::TS_BUCKETS; ++i) t.item0[i] = ch.ts_it[i] - ch.ts_it[0];
+    t.items_per_pos = ch.sper;
+    return t;
+  };
   auto plan64 = [&](const std::vector<int32_t>* list_in, int slot, std::vector<Chunk64>& chunks) -> int {
     chunks.clear();
     const int32_t m = list_in ? (int32_t)list_in->size() : nc;
@@ -1462,19 +1478,16 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       }
       // the chunked positions by column bucket (contiguous: sorted by column count, most first)
       ch.ts_pos[0] = ch.ne;
-      for (int i = 0; i < 3; ++i) {
+      for (int i = 0; i < rr::TS_BUCKETS; ++i) {
         int r = ch.ts_pos[i];
-        while (r < mc && rr::ts_bucket(kof(r)) == TS_NC[i]) ++r;
+        while (r < mc && rr::ts_list(kof(r)) == i) ++r;
         ch.ts_pos[i + 1] = r;
       }
-      if (ch.ts_pos[3] != mc) return fail(RR_E_ARG, "internal: chunked QR positions out of column order");
-      for (int i = 0; i < 4; ++i) ch.ts_it[i] = item_at(ch.ts_pos[i]);
+      if (ch.ts_pos[rr::TS_BUCKETS] != mc) return fail(RR_E_ARG, "internal: chunked QR positions out of column order");
+      for (int i = 0; i <= rr::TS_BUCKETS; ++i) ch.ts_it[i] = item_at(ch.ts_pos[i]);
       ch.ts_maxch = 0;
       for (int r = ch.ne; r < mc; ++r) ch.ts_maxch = std::max(ch.ts_maxch, item_at(r + 1) - item_at(r));
-      ch.ts_lw[0] = 0;
-      for (int i = 0; i < 3; ++i)
-        ch.ts_lw[i + 1] = ch.ts_lw[i] + (int64_t)(ch.ts_it[i + 1] - ch.ts_it[i]) * rr::ts_desc_words(TS_NC[i]);
-      max_lwords = std::max(max_lwords, ch.ts_lw[3]);
+      max_lwords = std::max(max_lwords, ts_list_words(ch));
       max_qpos = std::max<int64_t>(max_qpos, mc);
       max_qcol = std::max<int64_t>(max_qcol, (int64_t)ch.ne * ch.maxk);
       max_qpart = std::max<int64_t>(max_qpart, (int64_t)item_at(ch.ne) * 2 * ch.maxk);
@@ -1484,7 +1497,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     if (ctx->d_score_part.ensure((size_t)std::max<int64_t>(max_sitems, 1) * 8) != RR_OK) return RR_E_NOMEM;
     if (ctx->d_qst.ensure((size_t)std::max<int64_t>(max_qpos, 1) * sizeof(rr::QrState)) != RR_OK ||
         ctx->d_tsst.ensure((size_t)std::max<int64_t>(max_qpos, 1) * sizeof(rr::TsState)) != RR_OK ||
-        ctx->d_tslist.ensure((size_t)(max_lwords + 2) * 8) != RR_OK ||
+        ctx->d_tslist.ensure((size_t)max_lwords * 4) != RR_OK ||
         ctx->d_qphys.ensure((size_t)std::max<int64_t>(max_qcol, 1) * 4) != RR_OK ||
         ctx->d_qcold.ensure((size_t)std::max<int64_t>(max_qcol, 1) * 5 * 8) != RR_OK ||
         ctx->d_qpart.ensure((size_t)std::max<int64_t>(max_qpart, 1) * 8) != RR_OK)
@@ -1500,11 +1513,21 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     }
     // which unique factors a live candidate uses (after the factor-0 pre-pass)
     const int32_t nu = chunks.back().p0 + chunks.back().npair;
+    auto live_of = [&](const Chunk64& ch) {
+      return rr::LiveLaunch{(const int32_t*)ctx->d_f64_ord.p + ch.c0, dtab, dcds, ts_list(ch)};
+    };
     int pm = begin_phase(ctx, RR_PHASE_EVAL, stream);
-    RR_HIP(rr::launch_alive_fp64((const int32_t*)ctx->d_ustart.p, (const int32_t*)ctx->d_users.p, ddead, nu,
-                                 (int32_t*)ctx->d_alive.p, stream));
+    {   // with one launch chunk, its chunked QR's work lists in the same launch
+      const rr::LiveLaunch lv = live_of(chunks[0]);
+      RR_HIP(rr::launch_alive_fp64((const int32_t*)ctx->d_ustart.p, (const int32_t*)ctx->d_users.p, ddead, nu,
+                                   (int32_t*)ctx->d_alive.p, chunks.size() == 1 ? &lv : nullptr, stream));
+    }
     end_phase(ctx, pm, stream);
     for (const Chunk64& ch : chunks) {
+      if (chunks.size() > 1) {
+        const rr::LiveLaunch lv = live_of(ch);
+        RR_HIP(rr::launch_alive_fp64(nullptr, nullptr, ddead, 0, nullptr, &lv, stream));
+      }
       pm = begin_phase(ctx, RR_PHASE_EVAL, stream);
       if (ch.npair > 0) {
         rr::EvalLaunch E;
@@ -1553,11 +1576,9 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
         T.prog_kept = (const int64_t*)ctx->d_prog_kept.p;
         T.rp_off = (const int64_t*)ctx->d_rp_off.p + ch.c0;
         T.st = (rr::TsState*)ctx->d_tsst.p; T.rpart = (double*)ctx->d_slab.p;
-        // the work list: its three counters, then the descriptors
-        T.cnt = (int32_t*)ctx->d_tslist.p; T.desc = (int64_t*)ctx->d_tslist.p + 2;
-        for (int i = 0; i < 3; ++i) T.list_base[i] = ch.ts_lw[i];
+        T.list = ts_list(ch);
         RR_HIP(rr::launch_ts_init(T, ch.ne, mc, stream));
-        for (int i = 0; i < 3; ++i) RR_HIP(rr::launch_ts_chunk(T, i, ch.ts_it[i + 1] - ch.ts_it[i], stream));
+        for (int i = 0; i < rr::TS_BUCKETS; ++i) RR_HIP(rr::launch_ts_chunk(T, i, ch.ts_it[i + 1] - ch.ts_it[i], stream));
         RR_HIP(rr::launch_ts_solve(T, ch.ne, mc, ch.ts_maxch, stream));
       }
       end_phase(ctx, pm, stream);

@@ -64,14 +64,15 @@ struct QrLaunch {
 
 // Chunked column-pivoted QR of the FP64 OLS form, for candidates with at most
 // TS_MAX_COLS columns (free term included):
-//   launch_ts_init   one thread per position: the initial norms (from the
+//   launch_ts_init   one wave per position: the initial norms (from the
 //                    evaluation's chunk sums), the outcome when step 0 would
 //                    pivot a non-finite column, the finite columns, the rank
-//                    threshold; the chunk work items (position, chunk) of the
-//                    live positions appended to their column bucket's list;
-//   launch_ts_chunk  per bucket, a grid of workgroups over the bucket's list:
-//                    unpivoted Householder QR of a chunk of TS_ROWS rows of
-//                    [finite columns | y], its triangular factor to rpart;
+//                    threshold;
+//   launch_ts_chunk  per column bucket, a grid of workgroups over the chunk
+//                    work items of the bucket's live positions (the lists
+//                    launch_alive_fp64 wrote): unpivoted Householder QR of a
+//                    chunk of TS_ROWS rows of [finite columns | y], its
+//                    triangular factor to rpart;
 //   launch_ts_solve  the chunk factors combined in two levels -- one wave
 //                    per (position, group of TS_GROUP consecutive chunks)
 //                    folds the group's factors in chunk order into the slot
@@ -81,16 +82,38 @@ struct QrLaunch {
 //                    the step-synchronous QR).  max_chunks: the most chunks
 //                    of any position in the range.
 // Positions pos0..pos1-1 of the arrays (pointers not offset).  Column buckets
-// 0, 1, 2: 10, 5, 3 columns with y (ts_bucket).  Position p's chunk factors
-// sit at rpart + rp_off[p] + chunk * W, W = nc * (nc - 1) words for its
-// bucket's nc.  desc: the chunk work items, ts_desc_words(nc) words each
-// (factor address, rows, finite column count, the nc column addresses at the
-// chunk's first row), bucket b's from word list_base[b] on, room for as many
-// as its positions have chunks; cnt: 3 counters.
+// 0 .. 3: up to 10, 7, 5, 3 columns with y (ts_list).  Position p's chunk
+// factors sit at rpart + rp_off[p] + chunk * W, W = nc * (nc - 1) words, nc =
+// ts_bucket of its columns.
 constexpr int TS_MAX_COLS = 9;
 constexpr int64_t TS_ROWS = 4096;
 constexpr int TS_GRID = 2048;   // workgroups of a chunk launch at most
 constexpr int TS_GROUP = 16;    // chunks per group of the two-level combination
+constexpr int TS_BUCKETS = 4;   // column buckets of the chunk launches
+// The work lists of the chunk launches, of one launch chunk: the live
+// positions of each bucket (bucket b's at live + pos0[b], cnt[b] of them, in
+// position order).  A bucket's chunk work items are all chunks of its live
+// positions, chunk by chunk (items_per_pos > 0: every position has that many;
+// a chunk's columns, most of them shared by the candidates of a sweep, are
+// then read by all positions at about the same time), or, for positions of
+// several datasets, the (position, chunk) pairs at items + 2 item0[b],
+// cnt[TS_BUCKETS + b] of them, position p's from base[p] on.
+struct TsList {
+  int32_t* cnt;     // 2 TS_BUCKETS
+  int32_t* live;    // per position
+  int32_t* base;    // per position (items_per_pos == 0)
+  int32_t* items;   // 2 per chunk work item (items_per_pos == 0)
+  int32_t pos0[TS_BUCKETS + 1], item0[TS_BUCKETS];
+  int32_t items_per_pos;
+};
+// What launch_alive_fp64 needs to write one: the positions' candidates and
+// datasets.
+struct LiveLaunch {
+  const int32_t* order;
+  const DsDesc* ds;
+  const int32_t* cand_ds;
+  TsList list;
+};
 struct TsState {
   int32_t k, kf, size, live;            // live: 1 when the chunk and solve kernels have work
   int32_t fin[TS_MAX_COLS];             // the finite columns, in column order
@@ -118,22 +141,25 @@ struct TsLaunch {
   const int64_t* rp_off;      // per position: offset of its chunk factors in rpart
   TsState* st;
   double* rpart;
-  int32_t* cnt;
-  int64_t* desc;
-  int64_t list_base[3];
+  TsList list;
 };
 hipError_t launch_ts_init(const TsLaunch& L, int pos0, int pos1, hipStream_t s);
-// bucket 0, 1, 2; max_items: the bucket's chunk work items if every position
+// bucket 0 .. 3; max_items: the bucket's chunk work items if every position
 // were live
 hipError_t launch_ts_chunk(const TsLaunch& L, int bucket, int max_items, hipStream_t s);
 hipError_t launch_ts_solve(const TsLaunch& L, int pos0, int pos1, int64_t max_chunks, hipStream_t s);
-// the column count with y of the bucket of a candidate with k columns (free term included, k <= TS_MAX_COLS)
-__host__ __device__ inline int ts_bucket(int k) { return k <= 2 ? 3 : k <= 4 ? 5 : 10; }
-// words of a chunk work item's descriptor in the bucket of nc columns with y
-__host__ __device__ constexpr int ts_desc_words(int nc) { return 3 + nc; }
-// threads of the bucket's chunk sums (the order of the oracle's ts_dot): 256
+// the column count with y that fixes the order of the sums of a candidate
+// with k columns (free term included, k <= TS_MAX_COLS; the oracle's
+// ts_bucket), and the threads of that order (the oracle's ts_dot): 256
 // threads of 16 rows for 3 and 5 columns, 1024 of 4 rows for 10
+__host__ __device__ inline int ts_bucket(int k) { return k <= 2 ? 3 : k <= 4 ? 5 : 10; }
 __host__ __device__ constexpr int ts_threads(int nc) { return nc <= 5 ? 256 : 1024; }
+// the launch bucket of a candidate with k columns, the most columns with y it
+// takes, and its workgroup: the wide bucket is split so that a chunk of up to
+// 7 columns fits the registers of four waves (16 rows a thread); up to 10
+// take eight waves (8 rows a thread)
+__host__ __device__ inline int ts_list(int k) { return k >= 7 ? 0 : k >= 5 ? 1 : k >= 3 ? 2 : 3; }
+__host__ __device__ constexpr int ts_block(int nc) { return nc <= 7 ? 256 : 512; }
 
 // Scoring of the FP64 form: one workgroup per (launched position, chunk of
 // EVAL_CHUNK_ROWS rows) computes the chunk's sum of squared residuals --
@@ -223,9 +249,10 @@ hipError_t launch_qr_solve(const QrLaunch& L, hipStream_t s);
 hipError_t launch_qr_all1(const QrLaunch& L, hipStream_t s);
 hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s);
 // alive[u] = 1 if some candidate users[ustart[u] .. ustart[u+1]-1] has
-// dead == 0, else 0, for u < n
+// dead == 0, else 0, for u < n; live (or null): the work lists of a launch
+// chunk's chunked QR
 hipError_t launch_alive_fp64(const int32_t* ustart, const int32_t* users, const int32_t* dead, int32_t n,
-                             int32_t* alive, hipStream_t s);
+                             int32_t* alive, const LiveLaunch* live, hipStream_t s);
 // out[2f], out[2f+1]: sums of squares of feature f's column over rows >= 0
 // and rows >= 1 in the chunked order (rrm::chunk_sum)
 hipError_t launch_xnorm_fp64(const double* X, int64_t n, int64_t ldx, int32_t d, double* out, hipStream_t s);

@@ -43,6 +43,8 @@
 #include "rr_device.h"
 #include "rr_kernels.h"
 
+#include <type_traits>
+
 namespace rr {
 
 namespace {
@@ -1034,14 +1036,67 @@ __global__ __launch_bounds__(EV_THREADS, FORM == 0 ? 8 : R <= 2 ? 6 : 4) void k_
   }
 }
 
-// One thread per unique factor: whether a candidate still to be scored uses it.
-__global__ __launch_bounds__(256) void k_alive_fp64(const int32_t* ustart, const int32_t* users, const int32_t* dead,
-                                                    int32_t n, int32_t* alive) {
-  const int u = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (u >= n) return;
-  int32_t any = 0;
-  for (int32_t i = ustart[u]; i < ustart[u + 1] && !any; ++i) any = dead[users[i]] == 0;
-  alive[u] = any;
+// Blocks 0 .. alive_blocks-1: one thread per unique factor, whether a
+// candidate still to be scored uses it.  Then, if asked for, one block per
+// column bucket of the chunked QR: the bucket's live positions compacted in
+// position order (and the first chunk work item of each when the positions
+// have different numbers of chunks).  Counted here rather than by atomics of
+// k_ts_init's waves: no launch to clear counters (4.5 us a call), and k_ts_init
+// takes 20 us instead of 23 at 800 positions.
+constexpr int ALIVE_THREADS = 1024;
+__global__ __launch_bounds__(ALIVE_THREADS) void k_alive_fp64(const int32_t* ustart, const int32_t* users,
+                                                              const int32_t* dead, int32_t n, int32_t* alive,
+                                                              int alive_blocks, LiveLaunch lv) {
+  if ((int)blockIdx.x < alive_blocks) {
+    const int u = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (u >= n) return;
+    int32_t any = 0;
+    for (int32_t i = ustart[u]; i < ustart[u + 1] && !any; ++i) any = dead[users[i]] == 0;
+    alive[u] = any;
+    return;
+  }
+  constexpr int NW = ALIVE_THREADS / WAVE;
+  __shared__ int32_t wcnt[NW], wit[NW];
+  const int b = (int)blockIdx.x - alive_blocks;
+  const TsList& T = lv.list;
+  const int p1 = T.pos0[b + 1];
+  const int lane = (int)(threadIdx.x & (WAVE - 1)), wave = (int)(threadIdx.x / WAVE);
+  const bool items = T.items_per_pos == 0;
+  int32_t n_live = 0, n_items = 0;   // of the positions before this pass
+  for (int q = T.pos0[b]; q < p1; q += ALIVE_THREADS) {   // uniform
+    const int pos = q + (int)threadIdx.x;
+    int32_t it = 0;
+    bool in = false;
+    if (pos < p1) {
+      const int cand = lv.order[pos];
+      in = dead[cand] == 0;
+      if (in && items)
+        it = (int32_t)((lv.ds[lv.cand_ds ? lv.cand_ds[cand] : 0].n + TS_ROWS - 1) / TS_ROWS);
+    }
+    const uint64_t m = __ballot(in);
+    const int32_t before = __popcll(m & ((1ull << lane) - 1));
+    int32_t isum = it;   // inclusive scan over the wave
+    if (items) {
+      for (int s = 1; s < WAVE; s <<= 1) {
+        const int32_t o = __shfl_up(isum, s);
+        if (lane >= s) isum += o;
+      }
+    }
+    if (lane == WAVE - 1) { wcnt[wave] = __popcll(m); wit[wave] = isum; }
+    __syncthreads();
+    int32_t c0 = n_live, i0 = n_items;
+    for (int w = 0; w < NW; ++w) {
+      if (w < wave) { c0 += wcnt[w]; i0 += wit[w]; }
+      n_live += wcnt[w];
+      n_items += wit[w];
+    }
+    if (in) {
+      T.live[T.pos0[b] + c0 + before] = pos;
+      if (items) T.base[pos] = i0 + isum - it;
+    }
+    __syncthreads();   // wcnt and wit are reused
+  }
+  if (threadIdx.x == 0) { T.cnt[b] = n_live; T.cnt[TS_BUCKETS + b] = n_items; }
 }
 
 // Per feature of a dataset, the sums of squares of its column over rows >= 0
@@ -1331,10 +1386,8 @@ struct TsArgs {
   const int64_t* rp_off;
   TsState* st;
   double* rpart;
-  int32_t* ts_cnt;
-  int64_t* ts_desc;
-  int64_t list_base[3];
-  int pos0, pos1, bucket;
+  TsList list;
+  int pos0, bucket;
 };
 
 // Eigen's makeHouseholder (Householder.h:67-96) from the pivot c0 and the sum
@@ -1377,18 +1430,12 @@ __device__ inline void ts_factor(const TsArgs& a, const DsDesc& D, int pbeg, int
   *col = ts_col(a, D, pbeg, nf, j);
 }
 
-// One wave per position: a lane per factor finds its norm and column
-// (ts_factor, into fnd / fcol); lane 0 then does the position's work (outcome
-// of a non-finite step-0 pivot, finite columns, threshold, list slot); then
-// the wave writes the chunk work items' descriptors, a lane per chunk.
-__device__ inline bool ts_init_position(const TsArgs& a, int pos, int* slot_out, const double* fnd,
-                                        const double* const* fcol) {
+// Lane 0 of a position's wave: the outcome of a non-finite step-0 pivot, the
+// finite columns, the threshold, from the norms and columns in fnd / fcol.
+__device__ inline void ts_init_position(const TsArgs& a, int pos, int cand, const DsDesc& D, int pbeg, int nf,
+                                        const double* fnd, const double* const* fcol) {
   TsState& s = a.st[pos];
   s.live = 0;
-  const int cand = a.order[pos];
-  const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
-  const int pbeg = a.cand_start[cand];
-  const int nf = a.cand_start[cand + 1] - pbeg;
   const int k = nf + 1;
   const int64_t n = D.n;
   double nd[TS_MAX_COLS];
@@ -1408,7 +1455,7 @@ __device__ inline bool ts_init_position(const TsArgs& a, int pos, int* slot_out,
     for (int i = 0; i < size; ++i) co[i == 0 ? bi : (i == bi ? 0 : i)] = rrm::qnan();
     write_fit(a.fit + cand, rrm::qnan(), D.sst, n, size, 0);
     a.info[cand] = -1;
-    return false;
+    return;
   }
   int kf = 0;
   for (int j = 0; j < k; ++j)
@@ -1422,22 +1469,17 @@ __device__ inline bool ts_init_position(const TsArgs& a, int pos, int* slot_out,
   s.k = k;
   s.kf = kf;
   s.size = size;
-  const int nch = (int)((n + TS_ROWS - 1) / TS_ROWS);
-  s.nch = nch;
+  s.nch = (int)((n + TS_ROWS - 1) / TS_ROWS);
   s.n = n;
   s.live = 1;
-  const int nb = ts_bucket(k);
-  const int b = nb == 10 ? 0 : nb == 5 ? 1 : 2;
-  *slot_out = atomicAdd(a.ts_cnt + b, nch);
-  return true;
 }
 
+// One wave per position: a lane per factor finds its norm and column
+// (ts_factor), lane 0 does the position's work; for positions of several
+// datasets the wave also writes the position's (position, chunk) pairs, at
+// the offset its place in its bucket's list fixes.
 __global__ __launch_bounds__(WAVE) void k_ts_init(TsArgs a) {
   const int pos = a.pos0 + (int)blockIdx.x;
-  // what the other lanes need of lane 0's work, through LDS
-  __shared__ int live, slot, kf_s, nch_s, k_s;
-  __shared__ int64_t n_s;
-  __shared__ const double* col_s[TS_MAX_COLS + 1];
   __shared__ double fnd[TS_MAX_COLS];
   __shared__ const double* fcol[TS_MAX_COLS];
   const int cand = a.order[pos];
@@ -1445,44 +1487,16 @@ __global__ __launch_bounds__(WAVE) void k_ts_init(TsArgs a) {
     if (threadIdx.x == 0) a.st[pos].live = 0;
     return;
   }
-  {
-    const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
-    const int pbeg = a.cand_start[cand];
-    const int nf = a.cand_start[cand + 1] - pbeg;   // < TS_MAX_COLS
-    if ((int)threadIdx.x < nf) ts_factor(a, D, pbeg, nf, (int)threadIdx.x, &fnd[threadIdx.x], &fcol[threadIdx.x]);
-  }
+  const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
+  const int pbeg = a.cand_start[cand];
+  const int nf = a.cand_start[cand + 1] - pbeg;   // < TS_MAX_COLS
+  if ((int)threadIdx.x < nf) ts_factor(a, D, pbeg, nf, (int)threadIdx.x, &fnd[threadIdx.x], &fcol[threadIdx.x]);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int sl = 0;
-    live = ts_init_position(a, pos, &sl, fnd, fcol) ? 1 : 0;
-    slot = sl;
-    if (live) {
-      const TsState& s = a.st[pos];
-      kf_s = s.kf; nch_s = s.nch; k_s = s.k; n_s = s.n;
-      for (int f = 0; f <= s.kf; ++f) col_s[f] = s.col[f];
-    }
-  }
-  __syncthreads();
-  if (!live) return;   // uniform
-  // the position's chunk work items, appended to its bucket's list (the
-  // order of the list does not matter: every item writes its own factor) as
-  // self-contained descriptors: where its factor goes, its rows, its finite
-  // column count, its columns from the chunk's first row
-  const int kf = kf_s, nch = nch_s;
-  const int64_t n = n_s;
-  const int nb = ts_bucket(k_s);
-  const int b = nb == 10 ? 0 : nb == 5 ? 1 : 2;
-  const int dw = ts_desc_words(nb);
-  int64_t* const base = a.ts_desc + a.list_base[b] + (int64_t)slot * dw;
-  double* const out = a.rpart + a.rp_off[pos];
-  for (int c = (int)threadIdx.x; c < nch; c += WAVE) {
-    int64_t* const dst = base + (int64_t)c * dw;
-    const int64_t r0 = (int64_t)c * TS_ROWS;
-    dst[0] = (int64_t)(out + (int64_t)c * nb * (nb - 1));
-    dst[1] = (n - r0 < TS_ROWS) ? n - r0 : TS_ROWS;
-    dst[2] = kf;
-    for (int f = 0; f <= kf; ++f) dst[3 + f] = (int64_t)(col_s[f] + r0);
-  }
+  if (threadIdx.x == 0) ts_init_position(a, pos, cand, D, pbeg, nf, fnd, fcol);
+  if (a.list.items_per_pos > 0) return;
+  const int nch = (int)((D.n + TS_ROWS - 1) / TS_ROWS);
+  int32_t* const dst = a.list.items + 2 * ((int64_t)a.list.item0[ts_list(nf + 1)] + a.list.base[pos]);
+  for (int c = (int)threadIdx.x; c < nch; c += WAVE) { dst[2 * c] = pos; dst[2 * c + 1] = c; }
 }
 
 // A double moved between lanes by a DPP lane pattern (both halves).
@@ -1497,167 +1511,223 @@ __device__ inline double ts_readlane(double v, int lane) {
                           __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
-// Sum over the 64 lanes of a wave by the xor butterfly of strides 1, 2, 4,
-// ..., 32 (lane l adds lane l ^ s; a + b and b + a are the same bits, so every
-// lane of a combined group holds the same value): strides 1 and 2 by quad
-// permutations; then the groups of 4 and 8 are uniform, so stride 4 is the
-// mirror within 8 lanes and stride 8 the mirror within 16; strides 16 and 32
-// from lanes 0, 16, 32, 48.  Every thread gets the result.  All 64 lanes must
-// be active.
-__device__ inline double ts_wave_sum(double v) {
-  v = v + ts_dpp<0xB1>(v);    // quad_perm [1, 0, 3, 2]: lane ^ 1
-  v = v + ts_dpp<0x4E>(v);    // quad_perm [2, 3, 0, 1]: lane ^ 2
-  v = v + ts_dpp<0x141>(v);   // row_half_mirror: lane 7 - l of its 8
-  v = v + ts_dpp<0x140>(v);   // row_mirror: lane 15 - l of its 16
-  return (ts_readlane(v, 0) + ts_readlane(v, 16)) + (ts_readlane(v, 32) + ts_readlane(v, 48));
+// Sums over the 64 lanes of a wave of N values at once, each by the xor
+// butterfly of strides 1, 2, 4, ..., 32 (lane l adds lane l ^ s; a + b and
+// b + a are the same bits).  A plain butterfly computes every sum in every
+// lane.  Here lane pairs split the work: of two values a lane keeps one and
+// hands the other to its partner (a select each, one exchange, one addition
+// for both), so the values halve with every stride and N sums take about N +
+// 5 lane additions instead of 6 N.  Which of the two a lane keeps is the
+// stage's predicate, chosen so that partners differ in it and agree in all
+// earlier stages' predicates:
+//   stride 1   quad_perm [1,0,3,2]  (flips bit 0)       b0 ^ b2
+//   stride 2   quad_perm [2,3,0,1]  (flips bit 1)       b1 ^ b2
+//   stride 4   row_half_mirror      (flips bits 0-2)    b2 ^ b3
+//   stride 8   row_mirror           (flips bits 0-3)    b3
+//   stride 16  v_permlane16_swap    (exchanges rows)    b4
+//   stride 32  v_permlane32_swap    (exchanges halves)  b5
+// The mirrors stand for strides 4 and 8: within the groups below them one
+// lane of each group holds a value (lanes whose predicates agree), and the
+// mirror pairs those.  The swaps move both values at once and need no
+// select.  Value i ends in the lanes whose predicates spell i's bits
+// (TsLane::slot).  All 64 lanes must be active.
+struct TsLane {
+  bool k0, k1, k2, k3;
+  int slot;
+  __device__ explicit TsLane(int l)
+      : k0(((l ^ (l >> 2)) & 1) != 0), k1((((l >> 1) ^ (l >> 2)) & 1) != 0), k2((((l >> 2) ^ (l >> 3)) & 1) != 0),
+        k3(((l >> 3) & 1) != 0), slot((int)k0 | (int)k1 << 1 | (int)k2 << 2 | (l & 0x38)) {}
+};
+template <int STAGE, bool TWO>
+__device__ inline double ts_stage(const TsLane& L, double a, double b) {
+  if constexpr (STAGE >= 4) {
+    const double o = TWO ? b : a;
+    if constexpr (STAGE == 4) {
+      const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(o), false, false);
+      const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(o), false, false);
+      return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    } else {
+      const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(o), false, false);
+      const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(o), false, false);
+      return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    }
+  } else {
+    constexpr int CTRL = STAGE == 0 ? 0xB1 : STAGE == 1 ? 0x4E : STAGE == 2 ? 0x141 : 0x140;
+    if constexpr (!TWO) return a + ts_dpp<CTRL>(a);
+    const bool k = STAGE == 0 ? L.k0 : STAGE == 1 ? L.k1 : STAGE == 2 ? L.k2 : L.k3;
+    return (k ? b : a) + ts_dpp<CTRL>(k ? a : b);
+  }
+}
+// value I of those left after stages 0 .. K-1 of the N values f(0) .. f(N-1)
+// (depth first: few values are live at once)
+template <int K, int I, int N, class F>
+__device__ inline double ts_sums(const TsLane& L, const F& f) {
+  if constexpr (K == 0) {
+    return f(std::integral_constant<int, I>{});
+  } else {
+    constexpr int LEFT = (N + (1 << (K - 1)) - 1) >> (K - 1);   // values before this stage
+    const double a = ts_sums<K - 1, 2 * I, N>(L, f);
+    if constexpr (2 * I + 1 < LEFT) return ts_stage<K - 1, true>(L, a, ts_sums<K - 1, 2 * I + 1, N>(L, f));
+    else return ts_stage<K - 1, false>(L, a, a);
+  }
+}
+// the bits of a slot that tell N values apart
+constexpr int ts_slot_bits(int n) { return n <= 1 ? 0 : 1 + ts_slot_bits((n + 1) / 2); }
+
+template <int CT>
+struct TsLds {   // both halves are written in turn, by step
+  double prow[2][TS_MAX_COLS + 1];                 // the step's pivot row
+  double red[2][TS_MAX_COLS + 1][CT / WAVE + 2];   // group sums (padded: lane c reads row c)
+};
+
+// Step J of a chunk's QR (ts_chunk_item) and the ones after it.
+template <int J, int NC, int CT, int THR, int MR, bool FULL>
+__device__ inline void ts_chunk_steps(double (&v)[NC][MR], const TsLane& L, int m, int steps, TsLds<CT>& lds,
+                                      int& buf) {
+  if (J >= steps) return;   // uniform
+  constexpr int VG = CT / THR, VU = MR < VG ? MR : VG, LOGV = VU == 4 ? 2 : VU == 2 ? 1 : 0;
+  static_assert(VU == 1 << LOGV, "sum sets per thread");
+  constexpr int NW = THR / WAVE, N = (NC - J) * VU, BITS = ts_slot_bits(N);
+  const int t = (int)threadIdx.x;
+  const int lane = t & (WAVE - 1), wave = t / WAVE;
+  if (t == J) {
+#pragma unroll
+    for (int c = J; c < NC; ++c) lds.prow[buf][c] = v[c][0];
+  }
+  // partial sum of set S (the oracle's thread t + THR S) and column C
+  const double r = ts_sums<6, 0, N>(L, [&](auto ic) {
+    constexpr int S = ic.value & (VU - 1), C = J + (ic.value >> LOGV);
+    double s = 0.0;
+#pragma unroll
+    for (int i = S; i < MR; i += VG) {
+      const int row = t + THR * i;
+      if (FULL ? (i > 0 || t > J) : (row > J && row < m)) s = __builtin_fma(v[J][i], v[C][i], s);
+    }
+    return s;
+  });
+  const int sl = L.slot & ((1 << BITS) - 1);
+  if (sl < N && (L.slot >> BITS) == 0) lds.red[buf][J + (sl >> LOGV)][(sl & (VU - 1)) * NW + wave] = r;
+  __syncthreads();
+  // lane c: column c's group sums in order (groups of empty rows are zeros
+  // and are left out) and its reflector coefficients
+  const int c = lane < NC ? lane : NC - 1;
+  double tot = lds.red[buf][c][0];
+#pragma unroll
+  for (int g = 1; g < VU * NW; ++g) tot = tot + lds.red[buf][c][g];
+  const double pr = lds.prow[buf][c];
+  double beta, tau, den;
+  ts_householder(ts_readlane(pr, J), ts_readlane(tot, J), beta, tau, den);
+  if (__builtin_amdgcn_readfirstlane((int)(tau != 0.0))) {
+    const double w = pr + tot / den;
+    const double tw = tau * w;
+    const double g = tw / den;
+#pragma unroll
+    for (int q = J + 1; q < NC; ++q) {
+      // (both read before the rows part the lanes: the operand of a readlane
+      // in a branch is kept for the branch's lanes only)
+      const double gq = ts_readlane(g, q), twq = ts_readlane(tw, q);
+#pragma unroll
+      for (int i = 0; i < MR; ++i) {
+        const int row = t + THR * i;
+        if (i == 0 && t == J) v[q][i] = v[q][i] - twq;
+        else if (FULL ? (i > 0 || t > J) : (row > J && row < m)) v[q][i] = __builtin_fma(-v[J][i], gq, v[q][i]);
+      }
+    }
+  }
+  if (t == J) v[J][0] = beta;
+  buf ^= 1;   // the next step writes the other half; this one is read until its barrier
+  if constexpr (J + 2 < NC) ts_chunk_steps<J + 1, NC, CT, THR, MR, FULL>(v, L, m, steps, lds, buf);
 }
 
 // One chunk work item: unpivoted Householder QR of the chunk's [finite
-// columns | y] (m rows, kf finite columns), held in registers: thread t holds
-// rows t + THR u, u = 0 .. RPT-1.  Every sum is in the oracle's order for THR
-// threads: per thread its rows in order, groups of 64 by ts_wave_sum, the
-// group sums in order.  FULL: m == TS_ROWS, so only rows 0..j of step j
-// (thread t <= j, u = 0) need a condition.  The group sums go to LDS
-// (double-buffered by step parity, buf); with up to 4 groups every thread adds
-// them up itself (one barrier per step), with more one lane per column of
-// wave 0 adds them and the others read its totals (two barriers).
-template <int NC, int THR, bool FULL>
-__device__ inline void ts_chunk_item(const int64_t* cur, double (*prow)[NC], double (*red)[THR / WAVE][NC],
-                                     double (*totl)[NC], int& buf) {
-  constexpr int RPT = (int)(TS_ROWS / THR);
-  constexpr int NG = THR / WAVE;
+// columns | y] (m rows), held in registers: thread t of THR holds rows t +
+// THR i, i < MR (m <= THR MR).  Every sum is in the oracle's order for CT
+// threads (256 or 1024), CT / THR of them per thread here: its thread t + THR
+// s adds rows t + THR s, t + THR s + CT, ... in order; groups of 64 by
+// ts_sums; the group sums in order.  At most NC columns with y; columns past
+// the position's are zeros, which change nothing.  FULL: m == TS_ROWS, so
+// only rows 0..j of step j (i = 0) need a condition.
+// Per step: the partial sums of all columns reduced together, the group sums
+// to LDS, one barrier, then in every wave lane c adds up column c's group
+// sums and computes its reflector coefficients (one division sequence for
+// all columns), which the wave reads back as scalars.
+template <int NC, int CT, int THR, int MR, bool FULL>
+__device__ inline void ts_chunk_item(const TsState& st, int64_t r0, int m, double* out, int LD, TsLds<CT>& lds,
+                                     int& buf) {
   const int t = (int)threadIdx.x;
-  const int lane = t & (WAVE - 1), wave = t / WAVE;
-  double* const out = (double*)cur[0];
-  const int64_t m = cur[1];
-  const int kf = (int)cur[2];
-  const int nc = kf + 1;
-  double v[NC][RPT];
+  const int kf = st.kf, nc = kf + 1;
+  double v[NC][MR];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const double* src = c < nc ? (const double*)cur[3 + c] : nullptr;
+    if (c < nc) {   // uniform
+      const gcptr src = (gcptr)st.col[c] + r0;
 #pragma unroll
-    for (int u = 0; u < RPT; ++u) {
-      const int64_t row = t + (int64_t)THR * u;
-      v[c][u] = (src != nullptr && (FULL || row < m)) ? src[row] : 0.0;
-    }
-  }
-  const int steps = (int)((m < (int64_t)kf) ? m : (int64_t)kf);
-#pragma unroll
-  for (int j = 0; j < NC - 1; ++j) {
-    if (j >= steps) continue;   // uniform
-    if (t == j) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c) prow[buf][c] = v[c][0];
-    }
-    double ps[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) ps[c] = 0.0;
-#pragma unroll
-    for (int u = 0; u < RPT; ++u) {
-      const int64_t row = t + (int64_t)THR * u;
-      const bool in = FULL ? (u > 0 || t > j) : (row > j && row < m);
-      if (in) {
-        const double x = v[j][u];
-        ps[j] = __builtin_fma(x, x, ps[j]);
-#pragma unroll
-        for (int c = j + 1; c < NC; ++c)
-          if (c < nc) ps[c] = __builtin_fma(x, v[c][u], ps[c]);
-      }
-    }
-#pragma unroll
-    for (int c = j; c < NC; ++c)
-      if (c < nc) ps[c] = ts_wave_sum(ps[c]);
-    if (lane == 0) {
-#pragma unroll
-      for (int c = j; c < NC; ++c)
-        if (c < nc) red[buf][wave][c] = ps[c];
-    }
-    __syncthreads();
-    double tot[NC];
-    if constexpr (NG > 4) {
-      // many group sums: lane c of wave 0 adds column c's in group order and
-      // every thread reads the totals, instead of every thread adding them all
-      if (wave == 0 && lane >= j && lane < nc) {
-        double acc = red[buf][0][lane];
-#pragma unroll
-        for (int g = 1; g < NG; ++g) acc = acc + red[buf][g][lane];
-        totl[buf][lane] = acc;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int c = j; c < NC; ++c)
-        if (c < nc) tot[c] = totl[buf][c];
+      for (int i = 0; i < MR; ++i) v[c][i] = src[t + THR * i];   // whole chunks exist; rows past m are not used
     } else {
 #pragma unroll
-      for (int c = j; c < NC; ++c) {
-        if (c >= nc) continue;
-        double acc = red[buf][0][c];
-#pragma unroll
-        for (int g = 1; g < NG; ++g) acc = acc + red[buf][g][c];
-        tot[c] = acc;
-      }
+      for (int i = 0; i < MR; ++i) v[c][i] = 0.0;
     }
-    double beta, tau, den;
-    ts_householder(prow[buf][j], tot[j], beta, tau, den);
-    if (tau != 0.0) {
-#pragma unroll
-      for (int c = j + 1; c < NC; ++c) {
-        if (c >= nc) continue;
-        const double w = prow[buf][c] + tot[c] / den;
-        const double g = (tau * w) / den;
-#pragma unroll
-        for (int u = 0; u < RPT; ++u) {
-          const int64_t row = t + (int64_t)THR * u;
-          if (u == 0 && t == j) v[c][u] = v[c][u] - tau * w;
-          else if (FULL ? (u > 0 || t > j) : (row > j && row < m)) v[c][u] = __builtin_fma(-v[j][u], g, v[c][u]);
-        }
-      }
-    }
-    if (t == j) v[j][0] = beta;
-    buf ^= 1;   // the next step writes the other half; this one is read until its barrier
   }
+  const TsLane L(t & (WAVE - 1));
+  ts_chunk_steps<0, NC, CT, THR, MR, FULL>(v, L, m, m < kf ? m : kf, lds, buf);
   if (t < kf) {   // row t of the chunk's factor (rows past m are zero)
-    double* dst = out + (int64_t)t * NC;
+    double* dst = out + (int64_t)t * LD;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
-      if (c < nc) dst[c] = ((int64_t)t < m && c >= t) ? v[c][0] : 0.0;
+      if (c < nc) dst[c] = (t < m && c >= t) ? v[c][0] : 0.0;
   }
 }
+template <int NC, int CT, int THR>
+__device__ inline void ts_chunk_any(const TsState& st, int64_t r0, int m, double* out, int LD, TsLds<CT>& lds,
+                                    int& buf) {
+  constexpr int MR = (int)(TS_ROWS / THR);
+  if (m == TS_ROWS) ts_chunk_item<NC, CT, THR, MR, true>(st, r0, m, out, LD, lds, buf);
+  else if (m > THR) ts_chunk_item<NC, CT, THR, MR, false>(st, r0, m, out, LD, lds, buf);
+  else ts_chunk_item<NC, CT, THR, 1, false>(st, r0, m, out, LD, lds, buf);
+}
 
-// Chunk work items of the live positions, one bucket (positions with NC
-// columns with y) at a time: workgroups of ts_threads(NC) threads take items
-// blockIdx.x, blockIdx.x + gridDim.x, ... of the bucket's list (written by
-// k_ts_init) until the count is reached; the next item's descriptor is loaded
-// while the current one computes (up to 5 columns: the wide bucket has no
-// scalar registers to spare).
-template <int NC>
-__global__ __launch_bounds__(ts_threads(NC)) void k_ts_chunk(TsArgs a) {
-  constexpr int THR = ts_threads(NC);
-  constexpr int DW = ts_desc_words(NC);
-  constexpr bool PREFETCH = NC <= 5;
-  __shared__ double prow[2][NC];
-  __shared__ double red[2][THR / WAVE][NC];
-  __shared__ double totl[2][NC];
-  const int cnt = a.ts_cnt[a.bucket];   // uniform
-  const int64_t* const desc = a.ts_desc + a.list_base[a.bucket];
+// The chunk work items of one bucket's live positions (TsList): workgroups
+// take items blockIdx.x, blockIdx.x + gridDim.x, ...
+// Bound by instruction issue (reductions, reflector coefficients, updates) and
+// by the column reads, 9.7 TB/s out of the caches.  A sweep of 800 candidates
+// of 5 to 7 columns with y over 1e6 rows takes 3.46 ms; 8.91 ms with the
+// oracle's 1024 threads as the workgroup (4 rows each), plain butterflies and
+// every thread computing all coefficients: the reductions and the scalar work
+// ran in 16 waves per chunk instead of 4.  At 7500 rows 45 us instead of 98.
+template <int NCMAX>
+__global__ __launch_bounds__(ts_block(NCMAX), NCMAX <= 3 ? 3 : 2) void k_ts_chunk(TsArgs a) {
+  constexpr int CT = ts_threads(NCMAX), THR = ts_block(NCMAX);
+  constexpr int LD = NCMAX == 7 ? 10 : NCMAX;   // ts_bucket of its columns
+  __shared__ TsLds<CT> lds;
+  const TsList& T = a.list;
+  const int nlive = T.cnt[a.bucket], per = T.items_per_pos;
+  const int64_t total = per > 0 ? (int64_t)nlive * per : (int64_t)T.cnt[TS_BUCKETS + a.bucket];   // uniform
+  const int32_t* const live = T.live + T.pos0[a.bucket];
+  const int32_t* const pairs = T.items + 2 * (int64_t)T.item0[a.bucket];
   int buf = 0;   // LDS half of the next step
-  int item = (int)blockIdx.x;
-  if (item >= cnt) return;
-  int64_t cur[DW];
-#pragma unroll
-  for (int w = 0; w < DW; ++w) cur[w] = desc[(int64_t)item * DW + w];
-  for (;;) {
-    const int next = item + (int)gridDim.x;
-    int64_t nxt[DW];
-#pragma unroll
-    for (int w = 0; w < DW; ++w) nxt[w] = (PREFETCH && next < cnt) ? desc[(int64_t)next * DW + w] : 0;
-    if (cur[1] == TS_ROWS) ts_chunk_item<NC, THR, true>(cur, prow, red, totl, buf);
-    else ts_chunk_item<NC, THR, false>(cur, prow, red, totl, buf);
-    if (next >= cnt) break;
-    item = next;
-#pragma unroll
-    for (int w = 0; w < DW; ++w) cur[w] = PREFETCH ? nxt[w] : desc[(int64_t)item * DW + w];
+  for (int64_t item = (int64_t)blockIdx.x; item < total; item += (int64_t)gridDim.x) {
+    int pos, chunk;
+    if (per > 0) {
+      chunk = (int)(item / nlive);
+      pos = live[item - (int64_t)chunk * nlive];
+    } else {
+      pos = pairs[2 * item];
+      chunk = pairs[2 * item + 1];
+    }
+    const TsState& s = a.st[pos];
+    if (!s.live) continue;   // settled by k_ts_init
+    const int64_t r0 = (int64_t)chunk * TS_ROWS;
+    const int m = (int)(s.n - r0 < TS_ROWS ? s.n - r0 : TS_ROWS);
+    double* const out = a.rpart + a.rp_off[pos] + (int64_t)chunk * LD * (LD - 1);
+    const int nc = s.kf + 1;
+    if constexpr (NCMAX == 10) {
+      if (nc == 10) ts_chunk_any<10, CT, THR>(s, r0, m, out, LD, lds, buf);
+      else if (nc == 9) ts_chunk_any<9, CT, THR>(s, r0, m, out, LD, lds, buf);
+      else ts_chunk_any<8, CT, THR>(s, r0, m, out, LD, lds, buf);
+    } else {
+      if (nc == NCMAX) ts_chunk_any<NCMAX, CT, THR>(s, r0, m, out, LD, lds, buf);
+      else ts_chunk_any<NCMAX - 1, CT, THR>(s, r0, m, out, LD, lds, buf);
+    }
   }
 }
 
@@ -1845,10 +1915,6 @@ __global__ __launch_bounds__(WAVE) void k_ts_solve(TsArgs a) {
   }
 }
 
-__global__ void k_ts_zero(int32_t* cnt) {
-  if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
-}
-
 }  // namespace
 
 static QrArgs qr_args(const QrLaunch& L, int n_pos) {
@@ -1923,9 +1989,12 @@ hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s) {
 }
 
 hipError_t launch_alive_fp64(const int32_t* ustart, const int32_t* users, const int32_t* dead, int32_t n,
-                             int32_t* alive, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_alive_fp64, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ustart, users, dead, n, alive);
+                             int32_t* alive, const LiveLaunch* live, hipStream_t s) {
+  const unsigned nb = (unsigned)((n + ALIVE_THREADS - 1) / ALIVE_THREADS);
+  const unsigned blocks = nb + (live ? (unsigned)TS_BUCKETS : 0u);
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_alive_fp64, dim3(blocks), dim3(ALIVE_THREADS), 0, s, ustart, users, dead, n, alive, (int)nb,
+                     live ? *live : LiveLaunch{});
   return hipGetLastError();
 }
 
@@ -1984,32 +2053,31 @@ hipError_t launch_stats_fp64(const double* y, int64_t n, double* out4, hipStream
 }
 
 
-static TsArgs ts_args(const TsLaunch& L, int pos0, int pos1, int bucket) {
+static TsArgs ts_args(const TsLaunch& L, int pos0, int bucket) {
   return TsArgs{L.cand_start, L.prog_start, L.code, L.ds, L.cand_ds, L.coefs, L.fit, L.dead, L.info, L.order,
-                L.slab, L.norm_part, L.prog_item, L.prog_kept, L.rp_off, L.st, L.rpart, L.cnt, L.desc,
-                {L.list_base[0], L.list_base[1], L.list_base[2]}, pos0, pos1, bucket};
+                L.slab, L.norm_part, L.prog_item, L.prog_kept, L.rp_off, L.st, L.rpart, L.list, pos0, bucket};
 }
 
 hipError_t launch_ts_init(const TsLaunch& L, int pos0, int pos1, hipStream_t s) {
   if (pos1 <= pos0) return hipSuccess;
-  hipLaunchKernelGGL(k_ts_zero, dim3(1), dim3(WAVE), 0, s, L.cnt);
-  hipLaunchKernelGGL(k_ts_init, dim3((unsigned)(pos1 - pos0)), dim3(WAVE), 0, s, ts_args(L, pos0, pos1, 0));
+  hipLaunchKernelGGL(k_ts_init, dim3((unsigned)(pos1 - pos0)), dim3(WAVE), 0, s, ts_args(L, pos0, 0));
   return hipGetLastError();
 }
 
 hipError_t launch_ts_chunk(const TsLaunch& L, int bucket, int max_items, hipStream_t s) {
   if (max_items <= 0) return hipSuccess;
-  const TsArgs a = ts_args(L, 0, 0, bucket);
+  const TsArgs a = ts_args(L, 0, bucket);
   const dim3 grid((unsigned)(max_items < TS_GRID ? max_items : TS_GRID));
-  if (bucket == 2) hipLaunchKernelGGL(k_ts_chunk<3>, grid, dim3(ts_threads(3)), 0, s, a);
-  else if (bucket == 1) hipLaunchKernelGGL(k_ts_chunk<5>, grid, dim3(ts_threads(5)), 0, s, a);
-  else hipLaunchKernelGGL(k_ts_chunk<10>, grid, dim3(ts_threads(10)), 0, s, a);
+  if (bucket == 3) hipLaunchKernelGGL(k_ts_chunk<3>, grid, dim3(ts_block(3)), 0, s, a);
+  else if (bucket == 2) hipLaunchKernelGGL(k_ts_chunk<5>, grid, dim3(ts_block(5)), 0, s, a);
+  else if (bucket == 1) hipLaunchKernelGGL(k_ts_chunk<7>, grid, dim3(ts_block(7)), 0, s, a);
+  else hipLaunchKernelGGL(k_ts_chunk<10>, grid, dim3(ts_block(10)), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_ts_solve(const TsLaunch& L, int pos0, int pos1, int64_t max_chunks, hipStream_t s) {
   if (pos1 <= pos0) return hipSuccess;
-  const TsArgs a = ts_args(L, pos0, pos1, 0);
+  const TsArgs a = ts_args(L, pos0, 0);
   const int64_t groups = (max_chunks + TS_GROUP - 1) / TS_GROUP;
   if (groups > 65535) return hipErrorInvalidValue;
   if (max_chunks > 1)
