@@ -1558,7 +1558,9 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       if (ch.ne > 0) {
         Q.n_pos = ch.ne;
         if (ch.step_items[0] == ch.ne) {   // one chunk work item per position
-          RR_HIP(rr::launch_qr_all1(Q, stream));
+          int64_t n_max = 0;
+          for (size_t u = 0; u < uniq.size(); ++u) n_max = std::max(n_max, std::min(table[u].n, rr::EVAL_CHUNK_ROWS));
+          RR_HIP(rr::launch_qr_all1(Q, n_max, stream));
         } else {
           RR_HIP(rr::launch_qr_init(Q, stream));
           for (size_t st = 0; st < ch.step_pos.size(); ++st)

@@ -28,10 +28,57 @@ __device__ inline int64_t first_row(int64_t lo, int t) {
   return i < lo ? i + CP : i;
 }
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) v = v + __shfl_xor(v, s);
+// A double moved between lanes by a DPP lane pattern, or read from one lane.
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ inline double readlane_f64(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// The two halves (HALF) or neighbouring rows of 16 lanes of a and b exchanged:
+// lanes of the lower half (even rows) get a's own and a's from the other half,
+// lanes of the upper half (odd rows) b's from the other half and b's own.
+struct Swapped {
+  double x, y;
+};
+template <bool HALF>
+__device__ inline Swapped swap_f64(double a, double b) {
+  if constexpr (HALF) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return Swapped{__hiloint2double((int)hi[0], (int)lo[0]), __hiloint2double((int)hi[1], (int)lo[1])};
+  } else {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return Swapped{__hiloint2double((int)hi[0], (int)lo[0]), __hiloint2double((int)hi[1], (int)lo[1])};
+  }
+}
+// f over the 64 lanes by the butterfly of strides 32, 16, ..., 1 (f
+// commutative in bits; all 64 lanes active; every lane gets the result).  The
+// strides below 16 as rotations within the row: after stride 2s every lane
+// equals the one 2s away, so rotating by s finds the value of lane ^ s.  No
+// trip through the LDS crossbar as __shfl_xor would take.
+template <class F>
+__device__ inline double wave_fold(double v, F f) {
+  Swapped w = swap_f64<true>(v, v);
+  v = f(w.x, w.y);
+  w = swap_f64<false>(v, v);
+  v = f(w.x, w.y);
+  v = f(v, dpp_f64<0x128>(v));   // row_ror:8
+  v = f(v, dpp_f64<0x124>(v));   // row_ror:4
+  v = f(v, dpp_f64<0x122>(v));   // row_ror:2
+  v = f(v, dpp_f64<0x121>(v));   // row_ror:1
   return v;
+}
+__device__ inline double wave_sum(double v) {
+  return wave_fold(v, [](double a, double b) { return a + b; });
+}
+__device__ inline double wave_max(double v) {   // no NaN among the lanes
+  return wave_fold(v, [](double a, double b) { return a < b ? b : a; });
 }
 
 // Canonical block sums of NV values at once; every thread gets the results.

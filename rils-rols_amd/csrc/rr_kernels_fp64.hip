@@ -947,6 +947,230 @@ __global__ __launch_bounds__(QR_THREADS) void k_qr_all1(QrArgs a) {
   if (t0) qr_solve_pos(b, pos);
 }
 
+// Positions of one chunk whose columns fit LDS (ks <= WAVE columns, n <= 64 RG
+// rows): the whole step-synchronous QR with one workgroup per position and
+// its working columns in LDS.  A wave owns target columns: it computes a
+// column's dot product, top-row update, row updates, tail sums and norm
+// downdate by itself (the chunked order's groups of 64 rows one after the
+// other, lane l holding row 64 q + l), so a step has one barrier.  Every wave
+// carries the per-column arrays (norms, tail sums, permutation) of all
+// columns, lane j column j's, and makes the step's pivot choice and reflector
+// itself; a column's owner hands its new values to the others through LDS
+// (double-buffered by step).  Every value is computed by the operations of
+// qr_init_pos ... qr_solve_pos in their order.
+// Bound by the latency of a step's chain (pivot, square root, divisions, two
+// wave sums).  700 candidates of 14 columns on 150 rows: 75 us; with
+// k_qr_all1 (thread 0 alone on the serial parts, five barriers, the columns in global
+// memory) 270 us.
+constexpr int QS_THREADS = 512;
+constexpr size_t QS_LDS = 60 * 1024;   // for the columns, of the 64 KiB a workgroup may ask for
+// 12 WAVE rows of more than TS_MAX_COLS + 1 columns with y exceed QS_LDS
+static_assert((TS_MAX_COLS + 2) * 12 * WAVE * sizeof(double) > QS_LDS, "rows that fit LDS fit k_qr_small's registers");
+template <int RG>
+__global__ __launch_bounds__(QS_THREADS, 6) void k_qr_small(QrArgs a) {
+  constexpr int NW = QS_THREADS / WAVE, NQ = rrm::NORM_GROUPS;
+  extern __shared__ double qs_cols[];   // k + 1 columns (A, then y) of n rows
+  __shared__ double nu_s[2][WAVE], nd_s[2][WAVE], ts_s[2][WAVE], diag[WAVE];
+  const int pos = (int)blockIdx.x;
+  const int lane = (int)(threadIdx.x & (WAVE - 1)), wave = (int)(threadIdx.x / WAVE);
+  const int cand0 = a.order[pos];
+  if (a.dead && a.dead[cand0]) return;   // uniform
+  const Cand c = cand_of(a, pos);
+  const int k = c.k, nf = c.nf, n = (int)c.n;
+  const int size = n < k ? n : k;
+  double* const co = a.coefs + (int64_t)c.pbeg + c.cand;
+  // lane j: column j's source, norm and tail sum
+  const double* src = c.D->one;
+  double nd = __builtin_sqrt((double)n), ts = (double)(n - 1);
+  if (lane < nf) {
+    const int var = bare_variable(a.code + a.prog_start[c.pbeg + lane],
+                                  a.prog_start[c.pbeg + lane + 1] - a.prog_start[c.pbeg + lane]);
+    const double* const part = var >= 0 ? c.D->xnorm + 2 * var : a.norm_part + 2 * (int64_t)a.prog_item[c.pbeg + lane];
+    src = var >= 0 ? c.D->X + (int64_t)var * c.ldx : a.slab + a.prog_kept[c.pbeg + lane];
+    nd = __builtin_sqrt(part[0]);
+    ts = part[1];
+  }
+  {
+    const double s1 = readlane_f64(ts, 0);
+    if (nf > 0 && s1 != s1) {   // factor 0 NaN at a row >= 1 (qr_init_pos)
+      if (threadIdx.x == 0) {
+        for (int i = 0; i < k; ++i) co[i] = (i < size) ? rrm::qnan() : 0.0;
+        write_fit(a.fit + c.cand, rrm::qnan(), c.D->sst, c.n, size, 0);
+        a.info[c.cand] = -1;
+      }
+      return;
+    }
+  }
+  double nu = nd;
+  int phys = lane;
+  for (int col = wave; col <= k; col += NW) {
+    const uint64_t ad = (uint64_t)src;
+    const uint64_t sa = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ad, col & (WAVE - 1)) |
+                        (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(ad >> 32), col & (WAVE - 1)) << 32;
+    const gcptr from = (gcptr)(col < k ? (const double*)sa : c.D->y);
+    for (int i = lane; i < n; i += WAVE) qs_cols[col * n + i] = from[i];
+  }
+  // the largest of lanes p .. k-1 in the order of a left-to-right scan for a
+  // strictly greater value (a NaN never is; a NaN at p stays)
+  auto pivot = [&](int p, int* at) {
+    const double vp = readlane_f64(nu, p);
+    const bool in = lane >= p && lane < k && nu == nu;
+    const double m = wave_max(in ? nu : -__builtin_inf());
+    const uint64_t hit = __ballot(in && nu == m);
+    *at = (vp != vp || hit == 0) ? p : (int)__builtin_ctzll(hit);
+    return vp != vp ? vp : m;
+  };
+  int bi;
+  const double mx = pivot(0, &bi);
+  const double thr = ((mx * DBL_EPS) * (mx * DBL_EPS)) / (double)n;
+  __syncthreads();
+  int nonzero = size, steps = 0, buf = 0;
+  bool nan_out = false;
+  for (int p = 0; p < size; ++p) {   // every wave makes the same (uniform) decisions
+    const double best = pivot(p, &bi);
+    if (best * best < thr * (double)(n - p)) { nonzero = p; break; }
+    if (bi != p) {
+      const int other = lane == p ? bi : lane == bi ? p : lane;
+      nu = __shfl(nu, other);
+      nd = __shfl(nd, other);
+      ts = __shfl(ts, other);
+      phys = __shfl(phys, other);
+    }
+    const double* const v = qs_cols + __builtin_amdgcn_readlane(phys, p) * n;
+    const double c0 = v[p];
+    const double tail = (n - p == 1) ? 0.0 : readlane_f64(ts, p);
+    const bool zero_tail = tail <= DBL_MIN_;
+    double tau = 0.0, beta = c0;
+    if (!zero_tail) {
+      beta = __builtin_sqrt(c0 * c0 + tail);
+      if (c0 >= 0.0) beta = -beta;
+      tau = (beta - c0) / beta;
+      if (beta != beta && n - p > 1) {   // a NaN reflector (qr_begin_pos)
+        nan_out = true;
+        int r = size;
+        if (thr > 0.0) {
+          const uint64_t z = __ballot(lane > p && lane < size && nu == 0.0);
+          if (z) r = (int)__builtin_ctzll(z);
+        }
+        nonzero = r;
+        break;
+      }
+    }
+    if (threadIdx.x == 0) diag[p] = beta;
+    const int nrem = k - 1 - p;
+    steps = p + 1;
+    if (n - p == 1) break;   // a single row: its reflector is the identity (tau = 0)
+    const double den = c0 - beta;
+    const bool apply = tau != 0.0;
+    double e[RG];   // the essential part of the reflector
+#pragma unroll
+    for (int q = 0; q < RG; ++q) {
+      const int i = WAVE * q + lane;
+      e[q] = (apply && i > p && i < n) ? v[i] / den : 0.0;
+    }
+    for (int t = wave; t <= nrem; t += NW) {   // targets: positions p+1 .. k-1, then y
+      double* const x = qs_cols + (t < nrem ? __builtin_amdgcn_readlane(phys, p + 1 + t) : k) * n;
+      double xr[RG];
+#pragma unroll
+      for (int q = 0; q < RG; ++q) {
+        const int i = WAVE * q + lane;
+        xr[q] = (i > p && i < n) ? x[i] : 0.0;
+      }
+      double top = x[p];
+      if (apply) {
+        double acc[NQ];
+#pragma unroll
+        for (int g = 0; g < NQ; ++g) acc[g] = 0.0;
+#pragma unroll
+        for (int q = 0; q < RG; ++q) {
+          const int i = WAVE * q + lane;
+          if (i > p && i < n) acc[q % NQ] = acc[q % NQ] + e[q] * xr[q];
+        }
+        double sum = 0.0;
+#pragma unroll
+        for (int g = 0; g < NQ; ++g) {
+          if (g > 0 && WAVE * g >= n) continue;   // uniform: an empty group adds zero
+          const double s = wave_sum(acc[g]);
+          sum = g == 0 ? s : sum + s;
+        }
+        const double td = sum + top;
+        top = top - tau * td;
+        if (lane == 0) x[p] = top;
+        if (t == nrem && nrem == 0) continue;   // rows below p of Q^T y are never read
+#pragma unroll
+        for (int q = 0; q < RG; ++q) {
+          const int i = WAVE * q + lane;
+          if (i > p && i < n) {
+            const double te = tau * e[q];
+            xr[q] = xr[q] - te * td;
+            x[i] = xr[q];
+          }
+        }
+      }
+      if (t == nrem) continue;
+      double a1[NQ], a2[NQ];   // rows >= p+1, rows >= p+2
+#pragma unroll
+      for (int g = 0; g < NQ; ++g) a1[g] = a2[g] = 0.0;
+#pragma unroll
+      for (int q = 0; q < RG; ++q) {
+        const int i = WAVE * q + lane;
+        if (i > p && i < n) {
+          a1[q % NQ] = a1[q % NQ] + xr[q] * xr[q];
+          if (i >= p + 2) a2[q % NQ] = a2[q % NQ] + xr[q] * xr[q];
+        }
+      }
+      double s1 = 0.0, s2 = 0.0;
+#pragma unroll
+      for (int g = 0; g < NQ; ++g) {
+        if (g > 0 && WAVE * g >= n) continue;
+        const double u1 = wave_sum(a1[g]), u2 = wave_sum(a2[g]);
+        s1 = g == 0 ? u1 : s1 + u1;
+        s2 = g == 0 ? u2 : s2 + u2;
+      }
+      // the norm downdate (lawn_downdate_col)
+      const int j = p + 1 + t;
+      double nuj = readlane_f64(nu, j), ndj = readlane_f64(nd, j);
+      if (nuj != 0.0) {
+        double temp = __builtin_fabs(top) / nuj;
+        temp = (1.0 + temp) * (1.0 - temp);
+        temp = temp < 0.0 ? 0.0 : temp;
+        const double ratio = nuj / ndj;
+        const double temp2 = temp * (ratio * ratio);
+        if (temp2 <= __builtin_sqrt(DBL_EPS)) { ndj = nuj = __builtin_sqrt(s1); }
+        else nuj = nuj * __builtin_sqrt(temp);
+      }
+      if (lane == 0) { nu_s[buf][j] = nuj; nd_s[buf][j] = ndj; ts_s[buf][j] = s2; }
+    }
+    __syncthreads();
+    if (lane > p && lane < k) { nu = nu_s[buf][lane]; nd = nd_s[buf][lane]; ts = ts_s[buf][lane]; }
+    buf ^= 1;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  // back substitution (qr_solve_pos): lane i holds unknown i
+  const int r = nonzero;
+  double td = lane < r ? qs_cols[k * n + lane] : 0.0;
+  if (!nan_out) {
+    for (int i = r - 1; i >= 0; --i) {
+      const double ci = readlane_f64(td, i) / diag[i];
+      const double* const col = qs_cols + __builtin_amdgcn_readlane(phys, i) * n;
+      if (lane < i) td = td - ci * col[lane];
+      if (lane == i) td = ci;
+    }
+  }
+  const double cv = lane < r ? (nan_out || td != td ? rrm::qnan() : td) : 0.0;
+  if (lane < k) co[phys] = cv;
+  const bool any_nan = nan_out || __ballot(lane < k && cv != cv) != 0;
+  if (lane == 0) {
+    if (any_nan) {
+      write_fit(a.fit + c.cand, rrm::qnan(), c.D->sst, c.n, r, steps);
+      a.info[c.cand] = -1;
+    } else {
+      a.info[c.cand] = r | (steps << 16);
+    }
+  }
+}
+
 // Factor evaluation for the QR: one workgroup of EV_THREADS threads per
 // (unique factor, chunk of rrm::NORM_CHUNK rows).  A unique factor is one
 // program over one dataset, shared by every candidate of the launch that
@@ -1499,18 +1723,6 @@ __global__ __launch_bounds__(WAVE) void k_ts_init(TsArgs a) {
   for (int c = (int)threadIdx.x; c < nch; c += WAVE) { dst[2 * c] = pos; dst[2 * c + 1] = c; }
 }
 
-// A double moved between lanes by a DPP lane pattern (both halves).
-template <int CTRL>
-__device__ inline double ts_dpp(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-__device__ inline double ts_readlane(double v, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                          __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-
 // Sums over the 64 lanes of a wave of N values at once, each by the xor
 // butterfly of strides 1, 2, 4, ..., 32 (lane l adds lane l ^ s; a + b and
 // b + a are the same bits).  A plain butterfly computes every sum in every
@@ -1542,20 +1754,13 @@ template <int STAGE, bool TWO>
 __device__ inline double ts_stage(const TsLane& L, double a, double b) {
   if constexpr (STAGE >= 4) {
     const double o = TWO ? b : a;
-    if constexpr (STAGE == 4) {
-      const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(o), false, false);
-      const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(o), false, false);
-      return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-    } else {
-      const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(o), false, false);
-      const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(o), false, false);
-      return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-    }
+    const Swapped w = swap_f64<STAGE == 5>(a, o);
+    return w.x + w.y;
   } else {
     constexpr int CTRL = STAGE == 0 ? 0xB1 : STAGE == 1 ? 0x4E : STAGE == 2 ? 0x141 : 0x140;
-    if constexpr (!TWO) return a + ts_dpp<CTRL>(a);
+    if constexpr (!TWO) return a + dpp_f64<CTRL>(a);
     const bool k = STAGE == 0 ? L.k0 : STAGE == 1 ? L.k1 : STAGE == 2 ? L.k2 : L.k3;
-    return (k ? b : a) + ts_dpp<CTRL>(k ? a : b);
+    return (k ? b : a) + dpp_f64<CTRL>(k ? a : b);
   }
 }
 // value I of those left after stages 0 .. K-1 of the N values f(0) .. f(N-1)
@@ -1616,7 +1821,7 @@ __device__ inline void ts_chunk_steps(double (&v)[NC][MR], const TsLane& L, int 
   for (int g = 1; g < VU * NW; ++g) tot = tot + lds.red[buf][c][g];
   const double pr = lds.prow[buf][c];
   double beta, tau, den;
-  ts_householder(ts_readlane(pr, J), ts_readlane(tot, J), beta, tau, den);
+  ts_householder(readlane_f64(pr, J), readlane_f64(tot, J), beta, tau, den);
   if (__builtin_amdgcn_readfirstlane((int)(tau != 0.0))) {
     const double w = pr + tot / den;
     const double tw = tau * w;
@@ -1625,7 +1830,7 @@ __device__ inline void ts_chunk_steps(double (&v)[NC][MR], const TsLane& L, int 
     for (int q = J + 1; q < NC; ++q) {
       // (both read before the rows part the lanes: the operand of a readlane
       // in a branch is kept for the branch's lanes only)
-      const double gq = ts_readlane(g, q), twq = ts_readlane(tw, q);
+      const double gq = readlane_f64(g, q), twq = readlane_f64(tw, q);
 #pragma unroll
       for (int i = 0; i < MR; ++i) {
         const int row = t + THR * i;
@@ -1760,12 +1965,12 @@ __device__ inline void ts_fold_chain(double (&r)[TS_MAX_COLS], const double* src
       if (j >= kf) continue;   // uniform
       double tj[TS_MAX_COLS];   // T's column j, rows 0..j
 #pragma unroll
-      for (int i = 0; i <= j; ++i) tj[i] = ts_readlane(t[i], j);
+      for (int i = 0; i <= j; ++i) tj[i] = readlane_f64(t[i], j);
       double sxx = 0.0;
 #pragma unroll
       for (int i = 0; i <= j; ++i) sxx = __builtin_fma(tj[i], tj[i], sxx);
       double beta, tau, den;
-      ts_householder(ts_readlane(r[j], j), sxx, beta, tau, den);
+      ts_householder(readlane_f64(r[j], j), sxx, beta, tau, den);
       if (tau != 0.0 && l > j && l < nc) {
         double sx = 0.0;
 #pragma unroll
@@ -1954,8 +2159,15 @@ hipError_t launch_qr_step(const QrLaunch& L, int n_act, int n_items, hipStream_t
   return hipGetLastError();
 }
 
-hipError_t launch_qr_all1(const QrLaunch& L, hipStream_t s) {
+hipError_t launch_qr_all1(const QrLaunch& L, int64_t n_max, hipStream_t s) {
   if (L.n_pos <= 0) return hipSuccess;
+  const size_t cols = (size_t)(L.ks + 1) * (size_t)n_max * sizeof(double);
+  if (L.ks <= WAVE && cols <= QS_LDS) {
+    const QrArgs a = qr_args(L, L.n_pos);
+    if (n_max <= 4 * WAVE) hipLaunchKernelGGL(k_qr_small<4>, dim3((unsigned)L.n_pos), dim3(QS_THREADS), cols, s, a);
+    else hipLaunchKernelGGL(k_qr_small<12>, dim3((unsigned)L.n_pos), dim3(QS_THREADS), cols, s, a);
+    return hipGetLastError();
+  }
   const size_t lds = (size_t)L.ks * (7 * sizeof(double) + sizeof(int32_t));
   hipLaunchKernelGGL(k_qr_all1, dim3((unsigned)L.n_pos), dim3(QR_THREADS), lds, s, qr_args(L, L.n_pos));
   return hipGetLastError();

@@ -575,3 +575,44 @@ def test_repeated_candidates_take_the_same_results(ctx):
         assert fit[8].tobytes() == fit[10].tobytes()
     assert tuned[4]["factors"] != tuned[1]["factors"]
     ctx.free(h)
+
+
+# row groups of 64 and 256 around their edges, tables whose columns do and do
+# not fit a workgroup's LDS, one column a lane up to 64 and one more
+@pytest.mark.parametrize("n", [11, 64, 65, 150, 256, 257, 600, 700])
+def test_wide_candidates_of_small_tables_bitexact(ctx, n):
+    """The one-workgroup QR of wide candidates on small tables: coefficients
+    and rank of the oracle's QR over 10 to 66 columns, with columns that are
+    zero below row 0 or 1, repeated, constant, NaN or infinite among them."""
+    print("case: wide candidates of small tables n=%d" % n, flush=True)
+    rng = np.random.default_rng(290 + n)
+    X, y = make_data(290 + n, n, 5)
+    X[:, 3] = 0.0
+    X[0, 3] = 2.5
+    X[:, 4] = 0.0
+    X[:2, 4] = [1.5, -0.75]
+    pool = ["sin * x%d c0x%dp-1" % (i, m) for i in range(3) for m in range(1, 10)]
+    pool += ["exp * x%d c0x%dp-4" % (i, m) for i in range(3) for m in range(1, 10)]
+    pool += ["sqr x0", "sqr x1", "* x0 x1", "* x1 x2", "x0", "x1", "x2", "cos x0", "cos x1", "cos x2"]
+    special = ["x3", "x4", "+ x0 c0x0p+0", "x0", "c0x1.8p+1", "ln x1", "exp * x2 c0x1p+9"]
+    cands = []
+    for width in [9, 10, 13, 20, 63, 64, 65]:
+        for plain in (True, True, False, False, False):
+            f = [pool[i] for i in rng.choice(len(pool), min(width, len(pool)), replace=False)]
+            while len(f) < width:
+                f.append("sin + x0 c0x%dp+0" % len(f))
+            if not plain:
+                for s in rng.choice(len(special), 2, replace=False):
+                    f[int(rng.integers(1, width))] = special[s]
+            cands.append(f)
+    od = O.Dataset(X, y)
+    h = ctx.upload(X, y)
+    coefs, fit = ctx.fitness(h, capi.build_batch(cands), mode="ols")
+    alone = [ctx.fitness(h, capi.build_batch([f]), mode="ols") for f in cands]
+    ctx.free(h)
+    for f, c, ft, (ca, fa) in zip(cands, coefs, fit, alone):
+        o, rank = O.qr_solve(np.stack([od.eval(p) for p in f] + [np.ones(n)], axis=1), y)
+        assert same_bits(c, o), (len(f), f, c, o)
+        assert ft["rank"] == rank, (len(f), f)
+        assert same_bits(ca[0], o) and fa[0]["rank"] == rank, (len(f), f)
+        assert same_bits([ft["e0"], ft["e1"]], [fa[0]["e0"], fa[0]["e1"]]), (len(f), f)
