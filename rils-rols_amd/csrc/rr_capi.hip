@@ -1680,7 +1680,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     raw64.cand_ds = dcds; raw64.prog_kept = nullptr; raw64.order = nullptr; raw64.dead = nullptr; raw64.info = nullptr;
     raw64.pos_item = (const int32_t*)ctx->d_pos_item.p; raw64.n_pos = nc; raw64.n_items = (int)it;
     raw64.items_per_pos = per > 0 ? (int)per : 0; raw64.raw = 1;
-    raw64.rows = (int)ctx->fp64_eval_rows;
+    raw64.rows = (int)ctx->fp64_eval_rows; raw64.form = (int)ctx->fp64_eval_form; raw64.depth = batch_depth;
     raw64.part = (double*)ctx->d_score_part.p; raw64.fit = dfit;
   }
   if (checked && !list64.empty()) { if ((rc = plan64(&list64, 0, plan))) return rc; }

@@ -187,7 +187,7 @@ struct ScoreLaunch {
   int n_items;
   int items_per_pos;
   int raw;
-  int rows;                  // RAW: rows per thread per pass of the evaluation (1, 2, 4)
+  int rows, form, depth;     // RAW: as EvalLaunch's
   double* part;              // per work item
   rr_fit* fit;
 };

@@ -1202,8 +1202,9 @@ static_assert(EVAL_CHUNK_ROWS == rrm::NORM_CHUNK, "evaluation work items are the
 // fits in 64 VGPRs without new spills).  FORM 1: eval_lds_f64, the operand
 // stack in dynamic LDS (the launch's deepest program x R x EV_THREADS
 // doubles) and the transcendentals inlined.
+constexpr int eval_waves(int rows, int form) { return form == 0 ? 8 : rows <= 2 ? 6 : 4; }
 template <int R, int FORM>
-__global__ __launch_bounds__(EV_THREADS, FORM == 0 ? 8 : R <= 2 ? 6 : 4) void k_eval_fp64(EvalArgs a) {
+__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_eval_fp64(EvalArgs a) {
   static_assert(EV_THREADS == rrm::NORM_PARTIALS, "one thread per partial of the chunked order");
   __shared__ double red[EV_THREADS / WAVE][2];
   extern __shared__ double ev_stk[];
@@ -1438,9 +1439,14 @@ __device__ inline int score_pos(const ScoreArgs& a, int item) {
 // RAW: the tree (the candidate's one program) over the chunk; OLS: the OLS
 // tree's prediction from the coefficients and the factor columns, with the
 // arithmetic of tune_constants' tree (rils_rols_cpp.cpp:488-517).
-template <bool RAW, int R>
-__global__ __launch_bounds__(EV_THREADS, 8) void k_score_fp64(ScoreArgs a) {   // as k_eval_fp64
+// FORM as in k_eval_fp64, whose interpreters and register budgets these are.
+// RAW is bound by the evaluation's instruction issue: a call of 900 trees of
+// about 20 nodes on 50021 rows takes 713 us with the operand stack in LDS, 840
+// us with it in registers and the transcendentals called.
+template <bool RAW, int R, int FORM>
+__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_fp64(ScoreArgs a) {
   __shared__ double red[EV_THREADS / WAVE];
+  extern __shared__ double sc_stk[];   // RAW, FORM 1: the operand stack
   // OLS: per factor its column and coefficient; kind 0 skipped (|c| < 1e-12),
   // 1 the column itself (|c - 1| < 1e-12), 2 c times the column
   __shared__ const double* fcol[RAW ? 1 : RR_MAX_COLS];
@@ -1464,7 +1470,8 @@ __global__ __launch_bounds__(EV_THREADS, 8) void k_score_fp64(ScoreArgs a) {   /
     for (int64_t base = r0; base < r1; base += (int64_t)EV_THREADS * R) {   // rows < ldx
       const int64_t row0 = base + (int64_t)threadIdx.x;
       double v[R];
-      eval_f64<R, EV_THREADS>(code, len, a.K, D.X, ldx, row0, v);
+      if constexpr (FORM == 1) eval_lds_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v, sc_stk);
+      else eval_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int64_t i = row0 + (int64_t)EV_THREADS * r;
@@ -2180,15 +2187,20 @@ hipError_t launch_qr_solve(const QrLaunch& L, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Form 1's LDS stack: depth x rows x EV_THREADS doubles, within the 64 KiB a
+// workgroup may ask for; deeper launches take form 0.
+constexpr size_t EVAL_STACK_MAX = 65536;
+static size_t eval_stack(int depth, int rows) {
+  return (size_t)(depth > 0 ? depth : 1) * (size_t)rows * EV_THREADS * sizeof(double);
+}
+
 hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s) {
   if (L.n_items <= 0) return hipSuccess;
   EvalArgs a{L.prog_start, L.code,     L.K,        L.ds,       L.cand_ds, L.slab,          L.fac_prog,
              L.fac_cand,   L.fac_item, L.fac_kept, L.alive, L.n_facs,  L.items_per_fac, L.norm_part};
   const dim3 grid((unsigned)L.n_items), block(EV_THREADS);
-  // form 1's LDS stack: depth x rows x EV_THREADS doubles, within the 64 KiB
-  // a workgroup may ask for; deeper launches take form 0
-  const size_t stk = (size_t)(L.depth > 0 ? L.depth : 1) * (size_t)L.rows * EV_THREADS * sizeof(double);
-  if (L.form == 1 && stk <= 65536 && (L.rows == 1 || L.rows == 2 || L.rows == 4)) {
+  const size_t stk = eval_stack(L.depth, L.rows);
+  if (L.form == 1 && stk <= EVAL_STACK_MAX) {
     if (L.rows == 1) hipLaunchKernelGGL((k_eval_fp64<1, 1>), grid, block, stk, s, a);
     else if (L.rows == 4) hipLaunchKernelGGL((k_eval_fp64<4, 1>), grid, block, stk, s, a);
     else hipLaunchKernelGGL((k_eval_fp64<2, 1>), grid, block, stk, s, a);
@@ -2229,12 +2241,19 @@ hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {
               L.dead, L.info, L.pos_item, L.n_pos, L.items_per_pos, L.part, L.fit};
   const dim3 grid((unsigned)L.n_items), block(EV_THREADS), fgrid((unsigned)((L.n_pos + POS_THREADS - 1) / POS_THREADS));
   if (L.raw) {
-    if (L.rows == 1) hipLaunchKernelGGL((k_score_fp64<true, 1>), grid, block, 0, s, a);
-    else if (L.rows == 4) hipLaunchKernelGGL((k_score_fp64<true, 4>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_score_fp64<true, 2>), grid, block, 0, s, a);
+    const size_t stk = eval_stack(L.depth, L.rows);
+    if (L.form == 1 && stk <= EVAL_STACK_MAX) {
+      if (L.rows == 1) hipLaunchKernelGGL((k_score_fp64<true, 1, 1>), grid, block, stk, s, a);
+      else if (L.rows == 4) hipLaunchKernelGGL((k_score_fp64<true, 4, 1>), grid, block, stk, s, a);
+      else hipLaunchKernelGGL((k_score_fp64<true, 2, 1>), grid, block, stk, s, a);
+    } else {
+      if (L.rows == 1) hipLaunchKernelGGL((k_score_fp64<true, 1, 0>), grid, block, 0, s, a);
+      else if (L.rows == 4) hipLaunchKernelGGL((k_score_fp64<true, 4, 0>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((k_score_fp64<true, 2, 0>), grid, block, 0, s, a);
+    }
     hipLaunchKernelGGL(k_fit_fp64<true>, fgrid, dim3(POS_THREADS), 0, s, a);
   } else {
-    hipLaunchKernelGGL((k_score_fp64<false, 1>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_score_fp64<false, 1, 0>), grid, block, 0, s, a);
     hipLaunchKernelGGL(k_fit_fp64<false>, fgrid, dim3(POS_THREADS), 0, s, a);
   }
   return hipGetLastError();

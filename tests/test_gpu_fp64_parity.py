@@ -616,3 +616,27 @@ def test_wide_candidates_of_small_tables_bitexact(ctx, n):
         assert ft["rank"] == rank, (len(f), f)
         assert same_bits(ca[0], o) and fa[0]["rank"] == rank, (len(f), f)
         assert same_bits([ft["e0"], ft["e1"]], [fa[0]["e0"], fa[0]["e1"]]), (len(f), f)
+
+
+@pytest.mark.parametrize("form,rows", [(1, 1), (1, 2), (1, 4), (0, 2)])
+def test_raw_eval_forms_bitexact(ctx, form, rows):
+    """Raw scoring through both interpreters, over a ragged last chunk, with
+    programs of stack depth up to 4 (beyond form 1's LDS at 4 rows: form 0)."""
+    print("case: raw form %d rows=%d" % (form, rows), flush=True)
+    X, y = make_data(62, 9001, 4)
+    rng = np.random.default_rng(62)
+    trees = treegen.random_trees(62, 60, 1, 40, 4) + [_full_tree(rng, lv, 4) for lv in (2, 3, 4, 5, 6, 7)]
+    od = O.Dataset(X, y)
+    h = ctx.upload(X, y)
+    try:
+        ctx.set_option("fp64_eval_rows", rows)
+        ctx.set_option("fp64_eval_form", form)
+        for batch in (trees[:60], trees):
+            _, fit = ctx.fitness(h, capi.build_batch([[t] for t in batch]), mode="raw")
+            for t, f in zip(batch, fit):
+                e0, e1, _ = od.score(t)
+                assert same_bits([f["e0"], f["e1"]], [e0, e1]), t
+    finally:
+        ctx.set_option("fp64_eval_rows", 2)
+        ctx.set_option("fp64_eval_form", 1)
+    ctx.free(h)
