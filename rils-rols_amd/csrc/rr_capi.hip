@@ -1298,6 +1298,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       for (int32_t p = b->cand_start[c]; p < b->cand_start[c + 1]; ++p) {
         ph[p] = phash[p] ^ mx;
         bare[p] = is_bare(p);
+        if (bare[p]) prog_kept[p] = ~(int64_t)(b->code[b->prog_start[p]] >> 8);
       }
     }
     std::vector<int32_t> pfound(std::max(np, 1));   // phase 1: unique factor found in the chunk, or -1
@@ -1545,7 +1546,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       }
       end_phase(ctx, pm, stream);
       rr::QrLaunch Q{};
-      Q.cand_start = dc; Q.prog_start = dp; Q.code = dcode; Q.ds = dtab; Q.cand_ds = dcds;
+      Q.cand_start = dc; Q.ds = dtab; Q.cand_ds = dcds;
       Q.coefs = dcoef; Q.fit = dfit; Q.dead = ddead; Q.info = (int32_t*)ctx->d_info.p;
       Q.order = (const int32_t*)ctx->d_f64_ord.p + ch.c0; Q.slab = (double*)ctx->d_slab.p;
       Q.slab_off = (const int64_t*)ctx->d_f64_off.p + ch.c0;
@@ -1571,7 +1572,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       const int mc = ch.c1 - ch.c0;
       if (ch.ne < mc) {
         rr::TsLaunch T{};
-        T.cand_start = dc; T.prog_start = dp; T.code = dcode; T.ds = dtab; T.cand_ds = dcds;
+        T.cand_start = dc; T.ds = dtab; T.cand_ds = dcds;
         T.coefs = dcoef; T.fit = dfit; T.dead = ddead; T.info = (int32_t*)ctx->d_info.p;
         T.order = (const int32_t*)ctx->d_f64_ord.p + ch.c0; T.slab = (const double*)ctx->d_slab.p;
         T.norm_part = (const double*)ctx->d_norm_part.p; T.prog_item = (const int32_t*)ctx->d_prog_item.p;

@@ -38,8 +38,6 @@ struct QrState {
 };
 struct QrLaunch {
   const int32_t* cand_start;
-  const int32_t* prog_start;
-  const uint32_t* code;
   const DsDesc* ds;
   const int32_t* cand_ds;
   double* coefs;
@@ -54,7 +52,7 @@ struct QrLaunch {
   int n_pos;
   const double* norm_part;    // the evaluation's chunk sums (EvalLaunch::norm_part)
   const int32_t* prog_item;   // per non-bare program: the first evaluation work item of its factor
-  const int64_t* prog_kept;   // per non-bare program: slab offset of its factor's kept column
+  const int64_t* prog_kept;   // per program: slab offset of its factor's kept column, or ~v: the bare variable v
   QrState* st;
   int32_t* phys;
   double* cold;
@@ -125,8 +123,6 @@ struct TsState {
 };
 struct TsLaunch {
   const int32_t* cand_start;
-  const int32_t* prog_start;
-  const uint32_t* code;
   const DsDesc* ds;
   const int32_t* cand_ds;
   double* coefs;
@@ -161,13 +157,11 @@ __host__ __device__ constexpr int ts_threads(int nc) { return nc <= 5 ? 256 : 10
 __host__ __device__ inline int ts_list(int k) { return k >= 7 ? 0 : k >= 5 ? 1 : k >= 3 ? 2 : 3; }
 __host__ __device__ constexpr int ts_block(int nc) { return nc <= 7 ? 256 : 512; }
 
-// Scoring of the FP64 form: one workgroup per (launched position, chunk of
-// EVAL_CHUNK_ROWS rows) computes the chunk's sum of squared residuals --
-// RAW: of the candidate's one program; OLS: of the OLS tree from the
-// coefficients and the factor columns (kept slab columns, at slab +
-// prog_kept[program], or X), for the candidates whose info is >= 0 -- and
-// then one thread per position adds the
-// chunk sums in order and writes the fitness.  Position p owns work items
+// Scoring of the FP64 form: per (launched position, chunk of EVAL_CHUNK_ROWS
+// rows) the chunk's sum of squared residuals -- RAW: of the candidate's one
+// program; OLS: of the OLS tree from the coefficients and the factor columns
+// (prog_kept), for the candidates whose info is >= 0 -- and then per position
+// the chunk sums in order into the fitness.  Position p owns work items
 // pos_item[p] .. pos_item[p+1]-1 (items_per_pos > 0: p * items_per_pos ..).
 struct ScoreLaunch {
   const int32_t* cand_start;
@@ -178,7 +172,7 @@ struct ScoreLaunch {
   const int32_t* cand_ds;
   const double* coefs;       // OLS
   const double* slab;        // OLS
-  const int64_t* prog_kept;  // OLS, per non-bare program
+  const int64_t* prog_kept;  // OLS, per program (QrLaunch's)
   const int32_t* order;      // launched position -> candidate (null: identity)
   const int32_t* dead;       // or null
   const int32_t* info;       // OLS: written by the QR (k_ts_init / k_ts_solve, or k_qr_init / k_qr_solve)

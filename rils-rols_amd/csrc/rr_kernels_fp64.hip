@@ -43,6 +43,7 @@
 #include "rr_device.h"
 #include "rr_kernels.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace rr {
@@ -68,9 +69,10 @@ __device__ inline void write_fit(rr_fit* f, double ssr, double sst, int64_t n, i
   *f = o;
 }
 
-// Variable index of a program that is one LDV, else -1.
-__device__ inline int bare_variable(const uint32_t* code, int len) {
-  return (len == 1 && (code[0] & 0xffu) == RR_OP_LDV) ? (int)(code[0] >> 8) : -1;
+// Where a factor's values are: prog_kept of its program is the slab offset
+// of its kept column, or ~v for a program that is the bare variable v.
+__device__ inline const double* factor_col(int64_t kept, const double* slab, const DsDesc& D) {
+  return kept < 0 ? D.X + ~kept * D.ldx : slab + kept;
 }
 
 // ---------------------------------------------------------------- the QR
@@ -99,8 +101,6 @@ enum : int32_t { QF_DONE = 1, QF_PASS = 2, QF_APPLY = 4, QF_NOUPD = 8 };
 
 struct QrArgs {
   const int32_t* cand_start;
-  const int32_t* prog_start;
-  const uint32_t* code;
   const DsDesc* ds;
   const int32_t* cand_ds;
   double* coefs;
@@ -115,7 +115,7 @@ struct QrArgs {
   int n_pos;                 // positions taking part in this launch
   const double* norm_part;   // k_eval_fp64's chunk sums of squares
   const int32_t* prog_item;  // per non-bare program: its factor's first evaluation work item
-  const int64_t* prog_kept;  // per non-bare program: slab offset of its factor's kept column
+  const int64_t* prog_kept;  // per program: factor_col's
   QrState* st;
   int32_t* phys;             // per position: ks entries
   double* cold;              // normU, normD, tsq, cc, tdot: 5 blocks of (positions x ks)
@@ -147,10 +147,7 @@ __device__ inline Cand cand_of(const QrArgs& a, int pos) {
 // where the values of physical column col are before the first reflector:
 // the free term's ones, a bare variable's X column, or the kept column
 __device__ inline const double* origin_col(const QrArgs& a, const Cand& c, int col) {
-  if (col == c.nf) return c.D->one;
-  const int var = bare_variable(a.code + a.prog_start[c.pbeg + col],
-                                a.prog_start[c.pbeg + col + 1] - a.prog_start[c.pbeg + col]);
-  return var >= 0 ? c.D->X + (int64_t)var * c.ldx : a.slab + a.prog_kept[c.pbeg + col];
+  return col == c.nf ? c.D->one : factor_col(a.prog_kept[c.pbeg + col], a.slab, *c.D);
 }
 
 __device__ inline double* cold(const QrArgs& a, int which, int pos, int j) {
@@ -247,12 +244,11 @@ __device__ inline void qr_init_pos(const QrArgs& a, int pos) {
   const int64_t nch = (c.n + rrm::NORM_CHUNK - 1) / rrm::NORM_CHUNK;
   double* const co = a.coefs + (int64_t)c.pbeg + c.cand;
   for (int j = 0; j < c.nf; ++j) {
-    const int var = bare_variable(a.code + a.prog_start[c.pbeg + j],
-                                  a.prog_start[c.pbeg + j + 1] - a.prog_start[c.pbeg + j]);
+    const int64_t kept = a.prog_kept[c.pbeg + j];
     double s0, s1;
-    if (var >= 0) {
-      s0 = c.D->xnorm[2 * var];
-      s1 = c.D->xnorm[2 * var + 1];
+    if (kept < 0) {
+      s0 = c.D->xnorm[2 * ~kept];
+      s1 = c.D->xnorm[2 * ~kept + 1];
     } else {
       double s01[2];
       ordered_sums<2>(a.norm_part + 2 * (int64_t)a.prog_item[c.pbeg + j], 2, nch, s01);
@@ -388,7 +384,6 @@ __device__ inline const double* target_src(const QrArgs& a, int pos, const Cand&
 // are not used.  The columns are device memory: global address space.
 // (2 and 4 rows per step measure the same: the passes stream at the same
 // rate; 2 needs fewer registers)
-constexpr int QR_R = 4;       // rows per thread per step of the OLS scoring
 constexpr int QR_DOT_R = 2;   // ... of the dot pass
 constexpr int QR_UPD_R = 2;   // ... of the update pass
 typedef const __attribute__((address_space(1))) double* gcptr;
@@ -983,10 +978,9 @@ __global__ __launch_bounds__(QS_THREADS, 6) void k_qr_small(QrArgs a) {
   const double* src = c.D->one;
   double nd = __builtin_sqrt((double)n), ts = (double)(n - 1);
   if (lane < nf) {
-    const int var = bare_variable(a.code + a.prog_start[c.pbeg + lane],
-                                  a.prog_start[c.pbeg + lane + 1] - a.prog_start[c.pbeg + lane]);
-    const double* const part = var >= 0 ? c.D->xnorm + 2 * var : a.norm_part + 2 * (int64_t)a.prog_item[c.pbeg + lane];
-    src = var >= 0 ? c.D->X + (int64_t)var * c.ldx : a.slab + a.prog_kept[c.pbeg + lane];
+    const int64_t kept = a.prog_kept[c.pbeg + lane];
+    const double* const part = kept < 0 ? c.D->xnorm + 2 * ~kept : a.norm_part + 2 * (int64_t)a.prog_item[c.pbeg + lane];
+    src = factor_col(kept, a.slab, *c.D);
     nd = __builtin_sqrt(part[0]);
     ts = part[1];
   }
@@ -1403,9 +1397,9 @@ __global__ __launch_bounds__(NAN0_ROWS) void k_nan0_fp64(Nan0Args a) {
   }
 }
 
-// Scoring in the chunked order: work item b is chunk (b - pos_item[p]) of
-// launched position p (pos_item[p] <= b < pos_item[p+1]); items_per_pos > 0
-// when every position has that many (one dataset).
+// Scoring in the chunked order: position p owns work items pos_item[p] ..
+// pos_item[p+1]-1, one per chunk (items_per_pos > 0: every position has that
+// many, one dataset).
 struct ScoreArgs {
   const int32_t* cand_start;
   const int32_t* prog_start;
@@ -1415,20 +1409,22 @@ struct ScoreArgs {
   const int32_t* cand_ds;
   const double* coefs;
   const double* slab;
-  const int64_t* prog_kept;  // per non-bare program: slab offset of its factor's kept column
+  const int64_t* prog_kept;  // per program: factor_col's
   const int32_t* order;      // launched position -> candidate, or null (identity)
   const int32_t* dead;
   const int32_t* info;
   const int32_t* pos_item;
   int n_pos;
   int items_per_pos;
+  int span;                  // OLS, items_per_pos > 0: chunks per workgroup
   double* part;
   rr_fit* fit;
 };
 
+// the position of a work item of positions with different numbers of chunks:
+// the last whose first item is at or before it (uniform)
 __device__ inline int score_pos(const ScoreArgs& a, int item) {
-  if (a.items_per_pos > 0) return item / a.items_per_pos;
-  int lo = 0, hi = a.n_pos - 1;   // last position whose first item <= item (uniform)
+  int lo = 0, hi = a.n_pos - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (a.pos_item[mid] <= item) lo = mid; else hi = mid - 1;
@@ -1436,112 +1432,192 @@ __device__ inline int score_pos(const ScoreArgs& a, int item) {
   return lo;
 }
 
-// RAW: the tree (the candidate's one program) over the chunk; OLS: the OLS
-// tree's prediction from the coefficients and the factor columns, with the
-// arithmetic of tune_constants' tree (rils_rols_cpp.cpp:488-517).
-// FORM as in k_eval_fp64, whose interpreters and register budgets these are.
-// RAW is bound by the evaluation's instruction issue: a call of 900 trees of
-// about 20 nodes on 50021 rows takes 713 us with the operand stack in LDS, 840
-// us with it in registers and the transcendentals called.
-template <bool RAW, int R, int FORM>
-__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_fp64(ScoreArgs a) {
-  __shared__ double red[EV_THREADS / WAVE];
-  extern __shared__ double sc_stk[];   // RAW, FORM 1: the operand stack
-  // OLS: per factor its column and coefficient; kind 0 skipped (|c| < 1e-12),
-  // 1 the column itself (|c - 1| < 1e-12), 2 c times the column
-  __shared__ const double* fcol[RAW ? 1 : RR_MAX_COLS];
-  __shared__ double fcoef[RAW ? 1 : RR_MAX_COLS];
-  __shared__ int8_t fkind[RAW ? 1 : RR_MAX_COLS];
-  const int item = (int)blockIdx.x;
-  const int pos = score_pos(a, item);
-  const int cand = a.order ? a.order[pos] : pos;
-  if (a.dead && a.dead[cand]) return;   // uniform
-  if (!RAW && a.info[cand] < 0) return;
-  const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
-  const int64_t n = D.n, ldx = D.ldx;
-  const int64_t first = a.items_per_pos > 0 ? (int64_t)pos * a.items_per_pos : a.pos_item[pos];
-  const int64_t r0 = (item - first) * rrm::NORM_CHUNK;
-  const int64_t r1 = (r0 + rrm::NORM_CHUNK < n) ? r0 + rrm::NORM_CHUNK : n;
-  const int pbeg = a.cand_start[cand];
-  double s = 0.0;   // thread t: rows r0 + t (mod 256) in increasing order
-  if (RAW) {
-    const uint32_t* code = a.code + a.prog_start[pbeg];
-    const int len = a.prog_start[pbeg + 1] - a.prog_start[pbeg];
-    for (int64_t base = r0; base < r1; base += (int64_t)EV_THREADS * R) {   // rows < ldx
-      const int64_t row0 = base + (int64_t)threadIdx.x;
-      double v[R];
-      if constexpr (FORM == 1) eval_lds_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v, sc_stk);
-      else eval_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int64_t i = row0 + (int64_t)EV_THREADS * r;
-        if (i < r1) { const double d = D.y[i] - v[r]; s = s + d * d; }
-      }
-    }
-  } else {
-    const int nf = a.cand_start[cand + 1] - pbeg;
-    const double* co = a.coefs + (int64_t)pbeg + cand;
-    const double cf_free = co[nf];
-    for (int j = (int)threadIdx.x; j < nf; j += EV_THREADS) {
-      const double cj = co[j];
-      const uint32_t* code = a.code + a.prog_start[pbeg + j];
-      const int var = bare_variable(code, a.prog_start[pbeg + j + 1] - a.prog_start[pbeg + j]);
-      fcol[j] = var >= 0 ? D.X + (int64_t)var * ldx : a.slab + a.prog_kept[pbeg + j];
-      fcoef[j] = cj;
-      fkind[j] = (__builtin_fabs(cj) < EPS12) ? 0 : (__builtin_fabs(cj - 1) < EPS12) ? 1 : 2;
-    }
-    __syncthreads();
-    const gcptr yv = (gcptr)D.y;
-    // thread t: rows r0 + t (mod 256) in increasing order, QR_R at a time;
-    // rows at or beyond r1 read row r0 and are not added
-    for (int64_t base = r0; base < r1; base += (int64_t)EV_THREADS * QR_R) {
-      int64_t ii[QR_R];
-#pragma unroll
-      for (int r = 0; r < QR_R; ++r) {
-        const int64_t i = base + (int64_t)threadIdx.x + (int64_t)EV_THREADS * r;
-        ii[r] = i < r1 ? i : r0;
-      }
-      double yy[QR_R];   // issued with the first factor's loads: one wait per pass
-#pragma unroll
-      for (int r = 0; r < QR_R; ++r) yy[r] = yv[ii[r]];
-      double yp[QR_R], f[QR_R];
-      bool any = false;   // the same for every row
-      for (int j = 0; j < nf; ++j) {
-        const int kind = fkind[j];
-        if (kind == 0) continue;
-        const gcptr col = (gcptr)fcol[j];
-        const double cj = fcoef[j];
-#pragma unroll
-        for (int r = 0; r < QR_R; ++r) f[r] = col[ii[r]];
-#pragma unroll
-        for (int r = 0; r < QR_R; ++r) {
-          const double term = kind == 1 ? f[r] : cj * f[r];
-          yp[r] = any ? yp[r] + term : term;
-        }
-        any = true;
-      }
-      if (!(__builtin_fabs(cf_free) < EPS12)) {
-        const double term = cf_free * 1.0;
-#pragma unroll
-        for (int r = 0; r < QR_R; ++r) yp[r] = any ? yp[r] + term : term;
-        any = true;
-      }
-#pragma unroll
-      for (int r = 0; r < QR_R; ++r) {
-        if (base + (int64_t)threadIdx.x + (int64_t)EV_THREADS * r < r1) {
-          const double d = yy[r] - (any ? yp[r] : 0.0);
-          s = s + d * d;
-        }
-      }
-    }
-  }
+// The chunk's sum of squared residuals from the threads' partials; kept for
+// k_fit_fp64, or, where every position has one chunk, the fitness at once.
+// red is free again after the next barrier.
+__device__ inline void score_finish(const ScoreArgs& a, double s, double (&red)[EV_THREADS / WAVE], int64_t item,
+                                    const DsDesc& D, int cand, int32_t info) {
   s = wave_sum(s);
   if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = s;
   __syncthreads();
   if (threadIdx.x == 0) {
     double t = red[0];
     for (int w = 1; w < EV_THREADS / WAVE; ++w) t = t + red[w];
-    a.part[item] = t;
+    if (a.items_per_pos == 1) write_fit(a.fit + cand, t, D.sst, D.n, info & 0xffff, info >> 16);
+    else a.part[item] = t;
+  }
+}
+
+// RAW: one workgroup per work item, the candidate's one program over the chunk.
+// FORM as in k_eval_fp64, whose interpreters and register budgets these are.
+// Bound by the evaluation's instruction issue: a call of 900 trees of about 20
+// nodes on 50021 rows takes 713 us with the operand stack in LDS, 840 us with
+// it in registers and the transcendentals called.
+template <int R, int FORM>
+__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_raw(ScoreArgs a) {
+  __shared__ double red[EV_THREADS / WAVE];
+  extern __shared__ double sc_stk[];   // FORM 1: the operand stack
+  const int item = (int)blockIdx.x;
+  const int pos = a.items_per_pos > 0 ? item / a.items_per_pos : score_pos(a, item);
+  const int cand = a.order ? a.order[pos] : pos;
+  if (a.dead && a.dead[cand]) return;   // uniform
+  const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
+  const int64_t n = D.n, ldx = D.ldx;
+  const int64_t first = a.items_per_pos > 0 ? (int64_t)pos * a.items_per_pos : a.pos_item[pos];
+  const int64_t r0 = (item - first) * rrm::NORM_CHUNK;
+  const int64_t r1 = (r0 + rrm::NORM_CHUNK < n) ? r0 + rrm::NORM_CHUNK : n;
+  const int pbeg = a.cand_start[cand];
+  const uint32_t* code = a.code + a.prog_start[pbeg];
+  const int len = a.prog_start[pbeg + 1] - a.prog_start[pbeg];
+  double s = 0.0;   // thread t: rows r0 + t (mod 256) in increasing order
+  for (int64_t base = r0; base < r1; base += (int64_t)EV_THREADS * R) {   // rows < ldx
+    const int64_t row0 = base + (int64_t)threadIdx.x;
+    double v[R];
+    if constexpr (FORM == 1) eval_lds_f64<R, EV_THREADS>(code, len, a.K, D.X, ldx, row0, v, sc_stk);
+    else eval_f64<R, EV_THREADS>(code, len, a.K, D.X, ldx, row0, v);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t i = row0 + (int64_t)EV_THREADS * r;
+      if (i < r1) { const double d = D.y[i] - v[r]; s = s + d * d; }
+    }
+  }
+  score_finish(a, s, red, item, D, cand, 0);
+}
+
+// The OLS tree's prediction from the coefficients and the factor columns, with
+// the arithmetic of tune_constants' tree (rils_rols_cpp.cpp:488-517): terms
+// with |c| < 1e-12 dropped, the column itself where |c - 1| < 1e-12 (a
+// product by 1), the free term last, left to right.  The sum starts at -0.0,
+// which every term leaves as it is.
+constexpr int SC_NF = 8;   // factors whose columns are read together
+__device__ inline bool ols_skip(double c) { return __builtin_fabs(c) < EPS12; }
+__device__ inline double ols_coef(double c) { return __builtin_fabs(c - 1) < EPS12 ? 1.0 : c; }
+
+// The sum of squared residuals of this thread's rows of one chunk (thread t:
+// rows r0 + t mod 256 in increasing order); rows up to the chunk's end exist
+// in every column, those at or beyond m are not added.
+template <int NF>
+__device__ inline double score_rows(const gcptr (&col)[SC_NF], const double (&cf)[SC_NF], int skip, bool free_on,
+                                    double cf_free, gcptr yv, int64_t r0, int m) {
+  constexpr int R = NF <= 4 ? 4 : 2;   // rows per thread per pass: all loads of a pass are in flight together
+  double s = 0.0;
+  for (int base = 0; base < m; base += EV_THREADS * R) {
+    const int64_t row0 = r0 + base + (int64_t)threadIdx.x;
+    double yy[R], f[NF > 0 ? NF : 1][R], yp[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) { yy[r] = yv[row0 + EV_THREADS * r]; yp[r] = -0.0; }
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+#pragma unroll
+      for (int r = 0; r < R; ++r) f[j][r] = col[j][row0 + EV_THREADS * r];
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+      if (skip >> j & 1) continue;   // uniform
+#pragma unroll
+      for (int r = 0; r < R; ++r) yp[r] = yp[r] + cf[j] * f[j][r];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (free_on) yp[r] = yp[r] + cf_free;
+      if (base + (int)threadIdx.x + EV_THREADS * r < m) {
+        const double d = yy[r] - yp[r];
+        s = s + d * d;
+      }
+    }
+  }
+  return s;
+}
+
+// OLS: a workgroup scores span consecutive chunks of a position (1 for
+// positions of several datasets); the positions of one chunk group are
+// neighbouring workgroups, so the columns a sweep's candidates share are read
+// out of the L2 while they are there.  Up to SC_NF factors: addresses and
+// coefficients in scalar registers, every column's loads of a pass in flight
+// together; more: one column after the other.
+// Bound by the column reads: 800 candidates of 3 to 5 factors on 1e6 rows take
+// 1.20 ms, 5.6 GB of columns of their own and 30 GB of shared ones; position
+// by position with the columns looked up through the programs 2.30 ms.
+__global__ __launch_bounds__(EV_THREADS, 6) void k_score_ols(ScoreArgs a) {
+  __shared__ double red[2][EV_THREADS / WAVE];
+  const int b = (int)blockIdx.x;
+  int pos, c0, c1;
+  int64_t first;
+  if (a.items_per_pos > 0) {
+    const int g = b / a.n_pos;
+    pos = b - g * a.n_pos;
+    c0 = g * a.span;
+    c1 = min(c0 + a.span, a.items_per_pos);
+    first = (int64_t)pos * a.items_per_pos;
+  } else {
+    pos = score_pos(a, b);
+    first = a.pos_item[pos];
+    c0 = (int)(b - first);
+    c1 = c0 + 1;
+  }
+  const int cand = a.order[pos];
+  if (a.dead && a.dead[cand]) return;   // uniform
+  const int32_t info = a.info[cand];
+  if (info < 0) return;
+  const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
+  const int64_t n = D.n;
+  const int pbeg = a.cand_start[cand];
+  const int nf = a.cand_start[cand + 1] - pbeg;
+  const double* const co = a.coefs + (int64_t)pbeg + cand;
+  const double cf_free = readlane_f64(co[nf], 0);
+  const bool free_on = !ols_skip(cf_free);
+  const gcptr yv = (gcptr)D.y;
+  gcptr col[SC_NF];
+  double cf[SC_NF];
+  int skip = 0;
+  if (nf <= SC_NF) {
+    // lane j: factor j's coefficient and column, then read by lane
+    const int j = min((int)(threadIdx.x & (WAVE - 1)), max(nf - 1, 0));
+    const double cj = co[j];
+    const uint64_t ad = nf > 0 ? (uint64_t)factor_col(a.prog_kept[pbeg + j], a.slab, D) : 0;
+    skip = (int)__ballot(ols_skip(cj));
+    const double cm = ols_coef(cj);
+#pragma unroll
+    for (int q = 0; q < SC_NF; ++q) {
+      cf[q] = readlane_f64(cm, q);
+      col[q] = (gcptr)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ad, q) |
+                       (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(ad >> 32), q) << 32);
+    }
+  }
+  for (int c = c0; c < c1; ++c) {
+    const int64_t r0 = (int64_t)c * rrm::NORM_CHUNK;
+    const int m = (int)(n - r0 < rrm::NORM_CHUNK ? n - r0 : rrm::NORM_CHUNK);
+    double s = 0.0;
+    switch (nf) {   // uniform
+#define RR_NF(N) case N: s = score_rows<N>(col, cf, skip, free_on, cf_free, yv, r0, m); break;
+      RR_NF(0) RR_NF(1) RR_NF(2) RR_NF(3) RR_NF(4) RR_NF(5) RR_NF(6) RR_NF(7) RR_NF(8)
+#undef RR_NF
+      default: {
+        constexpr int R = 4;
+        for (int base = 0; base < m; base += EV_THREADS * R) {
+          const int64_t row0 = r0 + base + (int64_t)threadIdx.x;
+          double yp[R];
+#pragma unroll
+          for (int r = 0; r < R; ++r) yp[r] = -0.0;
+          for (int j = 0; j < nf; ++j) {
+            const double cj = co[j];
+            if (ols_skip(cj)) continue;
+            const gcptr x = (gcptr)factor_col(a.prog_kept[pbeg + j], a.slab, D);
+            const double cm = ols_coef(cj);
+#pragma unroll
+            for (int r = 0; r < R; ++r) yp[r] = yp[r] + cm * x[row0 + EV_THREADS * r];
+          }
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            if (free_on) yp[r] = yp[r] + cf_free;
+            if (base + (int)threadIdx.x + EV_THREADS * r < m) {
+              const double d = yv[row0 + EV_THREADS * r] - yp[r];
+              s = s + d * d;
+            }
+          }
+        }
+      }
+    }
+    score_finish(a, s, red[c & 1], first + c, D, cand, info);
   }
 }
 
@@ -1601,8 +1677,6 @@ __global__ __launch_bounds__(CP) void k_stats_fp64(const double* y, int64_t n, d
 // TsState; the chunk factors in rpart.
 struct TsArgs {
   const int32_t* cand_start;
-  const int32_t* prog_start;
-  const uint32_t* code;
   const DsDesc* ds;
   const int32_t* cand_ds;
   double* coefs;
@@ -1635,22 +1709,13 @@ __device__ inline void ts_householder(double c0, double tail_sq, double& beta, d
   }
 }
 
-// where physical column col of a candidate lives: the free term's ones, a
-// bare variable's X column, or the kept column of its factor
-__device__ inline const double* ts_col(const TsArgs& a, const DsDesc& D, int pbeg, int nf, int col) {
-  if (col == nf) return D.one;
-  const int var = bare_variable(a.code + a.prog_start[pbeg + col], a.prog_start[pbeg + col + 1] - a.prog_start[pbeg + col]);
-  return var >= 0 ? D.X + (int64_t)var * D.ldx : a.slab + a.prog_kept[pbeg + col];
-}
-
 // Factor j's column norm (from the evaluation's chunk sums, or the
 // dataset's feature norms for a bare variable) and where its column is.
-__device__ inline void ts_factor(const TsArgs& a, const DsDesc& D, int pbeg, int nf, int j, double* nd,
-                                 const double** col) {
-  const int var = bare_variable(a.code + a.prog_start[pbeg + j], a.prog_start[pbeg + j + 1] - a.prog_start[pbeg + j]);
+__device__ inline void ts_factor(const TsArgs& a, const DsDesc& D, int pbeg, int j, double* nd, const double** col) {
+  const int64_t kept = a.prog_kept[pbeg + j];
   double s0;
-  if (var >= 0) {
-    s0 = D.xnorm[2 * var];
+  if (kept < 0) {
+    s0 = D.xnorm[2 * ~kept];
   } else {
     const int64_t nch_eval = (D.n + rrm::NORM_CHUNK - 1) / rrm::NORM_CHUNK;
     double s01[2];
@@ -1658,7 +1723,7 @@ __device__ inline void ts_factor(const TsArgs& a, const DsDesc& D, int pbeg, int
     s0 = s01[0];
   }
   *nd = __builtin_sqrt(s0);
-  *col = ts_col(a, D, pbeg, nf, j);
+  *col = factor_col(kept, a.slab, D);
 }
 
 // Lane 0 of a position's wave: the outcome of a non-finite step-0 pivot, the
@@ -1721,7 +1786,7 @@ __global__ __launch_bounds__(WAVE) void k_ts_init(TsArgs a) {
   const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
   const int pbeg = a.cand_start[cand];
   const int nf = a.cand_start[cand + 1] - pbeg;   // < TS_MAX_COLS
-  if ((int)threadIdx.x < nf) ts_factor(a, D, pbeg, nf, (int)threadIdx.x, &fnd[threadIdx.x], &fcol[threadIdx.x]);
+  if ((int)threadIdx.x < nf) ts_factor(a, D, pbeg, (int)threadIdx.x, &fnd[threadIdx.x], &fcol[threadIdx.x]);
   __syncthreads();
   if (threadIdx.x == 0) ts_init_position(a, pos, cand, D, pbeg, nf, fnd, fcol);
   if (a.list.items_per_pos > 0) return;
@@ -2131,7 +2196,7 @@ __global__ __launch_bounds__(WAVE) void k_ts_solve(TsArgs a) {
 
 static QrArgs qr_args(const QrLaunch& L, int n_pos) {
   QrArgs a;
-  a.cand_start = L.cand_start; a.prog_start = L.prog_start; a.code = L.code; a.ds = L.ds; a.cand_ds = L.cand_ds;
+  a.cand_start = L.cand_start; a.ds = L.ds; a.cand_ds = L.cand_ds;
   a.coefs = L.coefs; a.fit = L.fit; a.dead = L.dead; a.info = L.info;
   a.order = L.order; a.slab = L.slab; a.slab_off = L.slab_off;
   a.pos_item = L.pos_item; a.items_per_pos = L.items_per_pos; a.n_pos = n_pos;
@@ -2237,24 +2302,34 @@ hipError_t launch_nan0_fp64(const Nan0Launch& L, hipStream_t s) {
 
 hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {
   if (L.n_pos <= 0) return hipSuccess;
+  // OLS: more chunks a workgroup once the launch is large, to spread a
+  // workgroup's setup (a chain of a few dependent loads).  800 candidates on
+  // 1e6 rows (196000 items): 1.23 ms at one chunk, 1.20 at five, 1.21 at eight;
+  // 4096 candidates on 1e5 rows (102400 items, five of six settled before):
+  // 125, 122 (three chunks) and 143 us (eight leave too few live workgroups)
+  const int span = L.items_per_pos > 0 ? std::max(1, std::min(8, L.n_items / 32768)) : 1;
   ScoreArgs a{L.cand_start, L.prog_start, L.code, L.K, L.ds, L.cand_ds, L.coefs, L.slab, L.prog_kept, L.order,
-              L.dead, L.info, L.pos_item, L.n_pos, L.items_per_pos, L.part, L.fit};
-  const dim3 grid((unsigned)L.n_items), block(EV_THREADS), fgrid((unsigned)((L.n_pos + POS_THREADS - 1) / POS_THREADS));
+              L.dead, L.info, L.pos_item, L.n_pos, L.items_per_pos, span, L.part, L.fit};
+  const dim3 block(EV_THREADS), fgrid((unsigned)((L.n_pos + POS_THREADS - 1) / POS_THREADS));
   if (L.raw) {
+    const dim3 grid((unsigned)L.n_items);
     const size_t stk = eval_stack(L.depth, L.rows);
     if (L.form == 1 && stk <= EVAL_STACK_MAX) {
-      if (L.rows == 1) hipLaunchKernelGGL((k_score_fp64<true, 1, 1>), grid, block, stk, s, a);
-      else if (L.rows == 4) hipLaunchKernelGGL((k_score_fp64<true, 4, 1>), grid, block, stk, s, a);
-      else hipLaunchKernelGGL((k_score_fp64<true, 2, 1>), grid, block, stk, s, a);
+      if (L.rows == 1) hipLaunchKernelGGL((k_score_raw<1, 1>), grid, block, stk, s, a);
+      else if (L.rows == 4) hipLaunchKernelGGL((k_score_raw<4, 1>), grid, block, stk, s, a);
+      else hipLaunchKernelGGL((k_score_raw<2, 1>), grid, block, stk, s, a);
     } else {
-      if (L.rows == 1) hipLaunchKernelGGL((k_score_fp64<true, 1, 0>), grid, block, 0, s, a);
-      else if (L.rows == 4) hipLaunchKernelGGL((k_score_fp64<true, 4, 0>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((k_score_fp64<true, 2, 0>), grid, block, 0, s, a);
+      if (L.rows == 1) hipLaunchKernelGGL((k_score_raw<1, 0>), grid, block, 0, s, a);
+      else if (L.rows == 4) hipLaunchKernelGGL((k_score_raw<4, 0>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((k_score_raw<2, 0>), grid, block, 0, s, a);
     }
-    hipLaunchKernelGGL(k_fit_fp64<true>, fgrid, dim3(POS_THREADS), 0, s, a);
   } else {
-    hipLaunchKernelGGL((k_score_fp64<false, 1, 0>), grid, block, 0, s, a);
-    hipLaunchKernelGGL(k_fit_fp64<false>, fgrid, dim3(POS_THREADS), 0, s, a);
+    const int64_t blocks = L.items_per_pos > 0 ? (int64_t)L.n_pos * ((L.items_per_pos + span - 1) / span) : L.n_items;
+    hipLaunchKernelGGL(k_score_ols, dim3((unsigned)blocks), block, 0, s, a);
+  }
+  if (L.items_per_pos != 1) {
+    if (L.raw) hipLaunchKernelGGL(k_fit_fp64<true>, fgrid, dim3(POS_THREADS), 0, s, a);
+    else hipLaunchKernelGGL(k_fit_fp64<false>, fgrid, dim3(POS_THREADS), 0, s, a);
   }
   return hipGetLastError();
 }
@@ -2285,7 +2360,7 @@ hipError_t launch_stats_fp64(const double* y, int64_t n, double* out4, hipStream
 
 
 static TsArgs ts_args(const TsLaunch& L, int pos0, int bucket) {
-  return TsArgs{L.cand_start, L.prog_start, L.code, L.ds, L.cand_ds, L.coefs, L.fit, L.dead, L.info, L.order,
+  return TsArgs{L.cand_start, L.ds, L.cand_ds, L.coefs, L.fit, L.dead, L.info, L.order,
                 L.slab, L.norm_part, L.prog_item, L.prog_kept, L.rp_off, L.st, L.rpart, L.list, pos0, bucket};
 }
 
