@@ -207,51 +207,33 @@ RR_HD inline double log(double x) {
 }
 
 // ---------------------------------------------------------------- sin / cos
-// 2/pi as a binary fraction, 64 bits per word, most significant first.
-RR_HD inline uint64_t two_over_pi_word(int i) {
-  switch (i) {
-    case 0: return 0xa2f9836e4e441529ULL;  case 1: return 0xfc2757d1f534ddc0ULL;
-    case 2: return 0xdb6295993c439041ULL;  case 3: return 0xfe5163abdebbc561ULL;
-    case 4: return 0xb7246e3a424dd2e0ULL;  case 5: return 0x06492eea09d1921cULL;
-    case 6: return 0xfe1deb1cb129a73eULL;  case 7: return 0xe88235f52ebb4484ULL;
-    case 8: return 0xe99c7026b45f7e41ULL;  case 9: return 0x3991d639835339f4ULL;
-    case 10: return 0x9c845f8bbdf9283bULL; case 11: return 0x1ff897ffde05980fULL;
-    case 12: return 0xef2f118b5a0a6d1fULL; case 13: return 0x6d367ecf27cb09b7ULL;
-    case 14: return 0x4f463f669e5fea2dULL; case 15: return 0x7527bac7ebe5f17bULL;
-    case 16: return 0x3d0739f78a5292eaULL; case 17: return 0x6bfb5fb11f8d5d08ULL;
-    case 18: return 0x56033046fc7b6babULL; case 19: return 0xf0cfbc209af4361dULL;
-    case 20: return 0xa9e391615ee61b08ULL; default: return 0x6599855f14a06840ULL;
-  }
-}
-
-// bits [pos, pos+64) of the 256-bit little-endian number r3:r2:r1:r0
-// (selects instead of array indexing so that no private memory is used)
-RR_HD inline uint64_t limb4(uint64_t r0, uint64_t r1, uint64_t r2, uint64_t r3, int i) {
-  return i == 0 ? r0 : i == 1 ? r1 : i == 2 ? r2 : i == 3 ? r3 : 0;
-}
-RR_HD inline uint64_t bits256(uint64_t r0, uint64_t r1, uint64_t r2, uint64_t r3, int pos) {
-  const int limb = pos >> 6, off = pos & 63;
-  uint64_t v = limb4(r0, r1, r2, r3, limb) >> off;
-  if (off != 0) v |= limb4(r0, r1, r2, r3, limb + 1) << (64 - off);
-  return v;
-}
+// (h:l) >> s, its low 64 bits, 0 <= s < 64
+RR_HD inline uint64_t funnel(uint64_t h, uint64_t l, int s) { return (l >> s) | ((h << 1) << (63 - s)); }
 
 // Payne-Hanek: |x| >= 2^28, finite.  Returns x = q pi/2 + (rh + rl).
+// On the GPU the lanes of a wavefront come with different exponents: the words
+// of 2/pi are a gather from a table in memory and every choice is a select or
+// a shift, 160 vector instructions.  As a switch the words were 8 trees of
+// branches, 1000 instructions when the lanes part: the evaluation of the
+// 4096-tree benchmark batch took 1303 us, 1284 us now.
 RR_HD inline void reduce_large(double ax, double* rh, double* rl, int* q) {
+  // 2/pi as a binary fraction, 64 bits per word, most significant first
+  static constexpr uint64_t TWO_OVER_PI_BITS[22] = {
+      0xa2f9836e4e441529ULL, 0xfc2757d1f534ddc0ULL, 0xdb6295993c439041ULL, 0xfe5163abdebbc561ULL,
+      0xb7246e3a424dd2e0ULL, 0x06492eea09d1921cULL, 0xfe1deb1cb129a73eULL, 0xe88235f52ebb4484ULL,
+      0xe99c7026b45f7e41ULL, 0x3991d639835339f4ULL, 0x9c845f8bbdf9283bULL, 0x1ff897ffde05980fULL,
+      0xef2f118b5a0a6d1fULL, 0x6d367ecf27cb09b7ULL, 0x4f463f669e5fea2dULL, 0x7527bac7ebe5f17bULL,
+      0x3d0739f78a5292eaULL, 0x6bfb5fb11f8d5d08ULL, 0x56033046fc7b6babULL, 0xf0cfbc209af4361dULL,
+      0xa9e391615ee61b08ULL, 0x6599855f14a06840ULL};
   const uint64_t u = d2bits(ax);
-  const int E = (int)((u >> 52) & 0x7ff) - 1075;            // ax = M 2^E
+  const int E = (int)((u >> 52) & 0x7ff) - 1075;            // ax = M 2^E, -24 <= E <= 971
   const uint64_t M = (u & 0x000fffffffffffffULL) | 0x0010000000000000ULL;
   const int s = (E - 1 > 1) ? E - 1 : 1;                     // first needed bit of 2/pi (1-based)
-  const int o = s - 1, wi = o >> 6, sh = o & 63;
-  const uint64_t w0 = two_over_pi_word(wi), w1 = two_over_pi_word(wi + 1);
-  const uint64_t w2 = two_over_pi_word(wi + 2), w3 = two_over_pi_word(wi + 3);
-  uint64_t W2, W1, W0;
-  if (sh == 0) { W2 = w0; W1 = w1; W0 = w2; }
-  else {
-    W2 = (w0 << sh) | (w1 >> (64 - sh));
-    W1 = (w1 << sh) | (w2 >> (64 - sh));
-    W0 = (w2 << sh) | (w3 >> (64 - sh));
-  }
+  const int o = s - 1, sh = o & 63;
+  const uint64_t* const w = TWO_OVER_PI_BITS + (o >> 6);      // words o/64 .. o/64 + 3, at most 18
+  const uint64_t W2 = (w[0] << sh) | ((w[1] >> 1) >> (63 - sh));
+  const uint64_t W1 = (w[1] << sh) | ((w[2] >> 1) >> (63 - sh));
+  const uint64_t W0 = (w[2] << sh) | ((w[3] >> 1) >> (63 - sh));
   unsigned __int128 t = (unsigned __int128)M * W0;
   const uint64_t r0 = (uint64_t)t;
   t = (unsigned __int128)M * W1 + (uint64_t)(t >> 64);
@@ -259,9 +241,13 @@ RR_HD inline void reduce_large(double ax, double* rh, double* rl, int* q) {
   t = (unsigned __int128)M * W2 + (uint64_t)(t >> 64);
   const uint64_t r2 = (uint64_t)t;
   const uint64_t r3 = (uint64_t)(t >> 64);
-  const int P = s + 191 - E;                                  // fractional bits of M*W
-  int qq = (int)(bits256(r0, r1, r2, r3, P) & 3);
-  uint64_t fh = bits256(r0, r1, r2, r3, P - 64), fl = bits256(r0, r1, r2, r3, P - 128);
+  // fractional bits of M*W: 190 where s = E - 1, else 192 - E <= 216, so the
+  // integer part starts in limb 2 or 3
+  const int P = s + 191 - E, off = P & 63;
+  const bool up = P >= 192;
+  const uint64_t l0 = up ? r1 : r0, l1 = up ? r2 : r1, l2 = up ? r3 : r2, l3 = up ? 0 : r3;
+  int qq = (int)(funnel(l3, l2, off) & 3);
+  uint64_t fh = funnel(l2, l1, off), fl = funnel(l1, l0, off);
   double sign = 1.0;
   if (fh >> 63) {                                             // fraction >= 1/2: use F - 1
     qq = (qq + 1) & 3;
