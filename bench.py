@@ -644,11 +644,13 @@ def executed_flops(factors, ks, E, flags, n, subset=None):
 def eval_kernel_flops(factors, flags, n):
     """Operators the FP64 evaluation kernel runs: every distinct non-bare factor
     of a candidate the pre-pass did not settle, once over all n rows (equal
-    factors share one evaluation)."""
+    factors share one evaluation), its constant subtrees folded as the FP64
+    form's programs have them."""
+    import rils_rols_cpp
     uniq = set()
     for c, fs in enumerate(factors):
         if not (int(flags[c]) & RR_F_EARLY):
-            uniq.update(f for f in fs if not BARE.match(f))
+            uniq.update(rils_rols_cpp._fold(f) for f in fs if not BARE.match(f))
     return float(n) * sum(ops_in(f) for f in uniq), len(uniq)
 
 

@@ -177,7 +177,7 @@ class BatchRunner {
     std::vector<int> nf;
     for (const std::string& t : trees) {
       rrh::ols_factors(rrh::parse_prefix(t), fs, pool);
-      for (const Flat& f : fs) { rrh::compile(f, code_, consts_); prog_.push_back((int32_t)code_.size()); }
+      for (const Flat& f : fs) add(f);
       cand_.push_back((int32_t)prog_.size() - 1);
       nf.push_back((int)fs.size());
     }
@@ -188,7 +188,7 @@ class BatchRunner {
     reset();
     mode_ = RR_MODE_OLS;
     for (const auto& c : cands) {
-      for (const std::string& f : c) { rrh::compile(rrh::parse_prefix(f), code_, consts_); prog_.push_back((int32_t)code_.size()); }
+      for (const std::string& f : c) add(rrh::parse_prefix(f));
       cand_.push_back((int32_t)prog_.size() - 1);
     }
   }
@@ -196,8 +196,7 @@ class BatchRunner {
     reset();
     mode_ = RR_MODE_RAW;
     for (const std::string& t : trees) {
-      rrh::compile(rrh::parse_prefix(t), code_, consts_);
-      prog_.push_back((int32_t)code_.size());
+      add(rrh::parse_prefix(t));
       cand_.push_back((int32_t)prog_.size() - 1);
     }
   }
@@ -208,7 +207,7 @@ class BatchRunner {
     py::array_t<double> coefs(std::max<int64_t>(ncoef, 1));
     py::array_t<double> fit({(py::ssize_t)std::max(nc, 1), (py::ssize_t)5});
     std::vector<rr_fit> out(std::max(nc, 1));
-    rr_batch b{nc, cand_.data(), prog_.data(), code_.data(), consts_.data(), (int32_t)consts_.size()};
+    rr_batch b = batch(pr);
     double* cp = (double*)coefs.request().ptr;
     {
       py::gil_scoped_release nogil;
@@ -236,7 +235,7 @@ class BatchRunner {
       cbuf[i].resize((size_t)std::max<int64_t>(ncoef, 1));
       fbuf[i].resize((size_t)std::max(nc, 1));
     }
-    rr_batch b{nc, cand_.data(), prog_.data(), code_.data(), consts_.data(), (int32_t)consts_.size()};
+    rr_batch b = batch(RR_FP64);
     std::vector<double> lat((size_t)k);
     std::vector<std::chrono::steady_clock::time_point> ts((size_t)k);
     double total = 0;
@@ -320,7 +319,7 @@ class BatchRunner {
   // the autotuner on the prepared batch; returns the best kernel time and the chosen options
   py::dict autotune(const std::string& precision, int reps) {
     const int pr = batch_precision(precision);
-    rr_batch b{(int32_t)cand_.size() - 1, cand_.data(), prog_.data(), code_.data(), consts_.data(), (int32_t)consts_.size()};
+    rr_batch b = batch(pr);
     double ms = 0;
     {
       py::gil_scoped_release nogil;
@@ -338,7 +337,23 @@ class BatchRunner {
 
  private:
   static void check(int rc, const char* what) { if (rc) throw std::runtime_error(std::string(what) + ": " + rr_last_error()); }
-  void reset() { cand_.assign(1, 0); prog_.assign(1, 0); code_.clear(); consts_.clear(); }
+  void reset() {
+    cand_.assign(1, 0); prog_.assign(1, 0); code_.clear(); consts_.clear();
+    prog64_.assign(1, 0); code64_.clear(); consts64_.clear();
+  }
+  void add(const Flat& f) {
+    rrh::compile(f, code_, consts_);
+    prog_.push_back((int32_t)code_.size());
+    rrh::compile_folded(f, code64_, consts64_, folder_);
+    prog64_.push_back((int32_t)code64_.size());
+  }
+  // the prepared batch: constants folded for the FP64 form
+  rr_batch batch(int precision) const {
+    const int32_t nc = (int32_t)cand_.size() - 1;
+    if (precision == RR_FP64)
+      return rr_batch{nc, cand_.data(), prog64_.data(), code64_.data(), consts64_.data(), (int32_t)consts64_.size()};
+    return rr_batch{nc, cand_.data(), prog_.data(), code_.data(), consts_.data(), (int32_t)consts_.size()};
+  }
   rr_ctx* ctx_ = nullptr;
   int32_t h_ = -1;
   int64_t n_ = 0;
@@ -347,6 +362,10 @@ class BatchRunner {
   std::vector<int32_t> cand_{0}, prog_{0}, scand_{0}, sprog_{0};
   std::vector<uint32_t> code_, scode_;
   std::vector<double> consts_;
+  std::vector<int32_t> prog64_{0};
+  std::vector<uint32_t> code64_;
+  std::vector<double> consts64_;
+  rrh::Folder folder_;
 };
 
 }  // namespace
@@ -497,6 +516,10 @@ PYBIND11_MODULE(rils_rols_cpp, m) {
   m.def("_relevant_features", &features_hook);
   m.def("_ols_factors", &factors_hook);
   m.def("_compile", &compile_hook);
+  m.def("_fold", [](const std::string& prefix) {
+    rrh::Folder folder;
+    return rrh::to_prefix(folder.fold(rrh::parse_prefix(prefix)));
+  });
   m.def("_ols_tree", &ols_tree_hook);
   m.def("_crand", &rand_hook);
 }

@@ -96,8 +96,11 @@ class GpuSession {
     std::vector<int32_t> cand_start{0}, prog_start{0};
     std::vector<uint32_t> code;
     std::vector<double> consts;
+    Folder folder;
+    bool fold = true;   // FP64 batches
     void add(const Flat& f) {
-      compile(f, code, consts);
+      if (fold) compile_folded(f, code, consts, folder);
+      else compile(f, code, consts);
       prog_start.push_back((int32_t)code.size());
     }
     void close_candidate() { cand_start.push_back((int32_t)prog_start.size() - 1); }
@@ -139,6 +142,7 @@ class GpuSession {
   void ols_subset(const std::vector<std::vector<Flat>>& factors, const int32_t* idx, size_t count, int precision,
                   std::vector<double>& coefs, std::vector<int64_t>& off, std::vector<rr_fit>& out, Stats& st) {
     Builder B;
+    B.fold = precision == RR_FP64;
     off.resize(count);
     int64_t total = 0;
     for (size_t q = 0; q < count; ++q) {

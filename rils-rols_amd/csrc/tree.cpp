@@ -1,6 +1,9 @@
 // tree.cpp -- host-side expression engine (see tree.h).
 #include "tree.h"
 
+#define RR_HD
+#include "rr_math.h"
+
 #include <charconv>
 
 #include <climits>
@@ -429,6 +432,61 @@ int ols_tree_size(const std::vector<int32_t>& fs, const double* coefs) {
   return sz + kept - 1;
 }
 
+// ---- constant folding
+// 4096 random trees of 3 to 50 nodes over 1e5 rows (half of their leaves
+// constants): four tenths of the estimated evaluation work reads no variable;
+// of a local-search sweep's factors and of its whole trees about a sixth.
+const Flat& Folder::fold(const Flat& f) {
+  bool any = false;
+  for (size_t i = 0; i + 1 < f.size() && !any; ++i)
+    any = arity(f[i].t) == 1 ? f[i + 1].t == CONST
+                             : arity(f[i].t) == 2 && f[i + 1].t == CONST && i + 2 < f.size() && f[i + 2].t == CONST;
+  if (!any) return f;   // every constant subtree holds one whose operands are all constants
+  rev_.clear();
+  st_.clear();
+  for (size_t i = f.size(); i-- > 0;) {   // operands before operators, the tokens in reverse
+    const Tok& t = f[i];
+    const int a = arity(t.t);
+    if (a == 0) {
+      st_.push_back(Ent{t.t == CONST, t.c, rev_.size()});
+      rev_.push_back(t);
+      continue;
+    }
+    const Ent l = st_.back();
+    st_.pop_back();
+    Ent r = l;   // the right operand came first
+    if (a == 2) { r = st_.back(); st_.pop_back(); }
+    Ent e{l.cst && r.cst && t.t != POW, 0.0, r.start};
+    if (e.cst) {
+      switch (t.t) {
+        case PLUS: e.v = l.v + r.v; break;
+        case MINUS: e.v = l.v - r.v; break;
+        case MULTIPLY: e.v = l.v * r.v; break;
+        case DIVIDE: e.v = l.v / r.v; break;
+        case LT: e.v = l.v < r.v ? 1.0 : 0.0; break;
+        case GT: e.v = l.v > r.v ? 1.0 : 0.0; break;
+        case EQ: e.v = l.v == r.v ? 1.0 : 0.0; break;
+        case NEQ: e.v = l.v != r.v ? 1.0 : 0.0; break;
+        case MIN: e.v = l.v < r.v ? l.v : r.v; break;
+        case MAX: e.v = l.v > r.v ? l.v : r.v; break;
+        case SIN: e.v = rrm::sin(l.v); break;
+        case COS: e.v = rrm::cos(l.v); break;
+        case LN: e.v = rrm::log(l.v); break;
+        case EXP: e.v = rrm::exp(l.v); break;
+        case SQRT: e.v = rrm::sqrt(l.v); break;
+        default: e.v = l.v * l.v; break;   // SQR
+      }
+      rev_.resize(e.start);
+      rev_.push_back(tok_const(e.v));
+    } else {
+      rev_.push_back(t);
+    }
+    st_.push_back(e);
+  }
+  out_.assign(rev_.rbegin(), rev_.rend());
+  return out_;
+}
+
 // ---- bytecode
 namespace {
 struct Emitter {
@@ -497,6 +555,18 @@ struct Emitter {
   }
 };
 }  // namespace
+
+void compile_folded(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts, Folder& folder) {
+  const Flat& g = folder.fold(f);
+  if (&g != &f && f.size() >= ((size_t)2 << RR_MAX_STACK) - 1) {
+    // large enough for the unfolded program to need too many stack slots:
+    // what compile() refuses is refused here
+    std::vector<uint32_t> c;
+    std::vector<double> k;
+    compile(f, c, k);
+  }
+  compile(g, code, consts);
+}
 
 int compile(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts) {
   std::vector<int32_t> sz;

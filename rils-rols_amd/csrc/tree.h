@@ -97,8 +97,25 @@ struct Program {
   std::vector<uint32_t> code;
   int depth = 0;
 };
+// Constant folding for the FP64 form: every subtree that reads no variable
+// becomes the constant it evaluates to, by the operations the device would
+// carry out in every row (rr_math.h gives the same bits on the host), so the
+// program's values keep their bits.  Not for the FP32 form, whose bounds and
+// certificates are those of its own evaluation of the constants.
+class Folder {
+ public:
+  // f itself when there is nothing to fold, else a tree valid until the next call
+  const Flat& fold(const Flat& f);
+ private:
+  struct Ent { bool cst; double v; size_t start; };   // a subtree: its tokens in rev_ begin at start
+  Flat rev_, out_;
+  std::vector<Ent> st_;
+};
+
 // Appends the program of subtree `f` to `code`, its constants to `consts`.
 // Returns the operand-stack depth it needs.
 int compile(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts);
+// The same for the FP64 form: the program of the folded tree.
+void compile_folded(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts, Folder& folder);
 
 }  // namespace rrh

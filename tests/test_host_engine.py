@@ -86,6 +86,33 @@ def test_compile_matches_test_compiler():
         assert np.array_equal(np.array(consts), arrs["consts"][:arrs["n_consts"]]), t
 
 
+def test_folded_constants_keep_the_values():
+    """A folded tree has no operator over constants left and evaluates to the
+    same bits as the tree itself (a NaN of either sign is a NaN)."""
+    rng = np.random.default_rng(5)
+    X = np.concatenate([rng.uniform(-5, 5, (200, 5)), [[0.0, -0.0, 1.0, -1.0, 2.0], [1e300, -1e300, np.inf, 0.5, 3.0]]])
+    od = O.Dataset(X, np.zeros(len(X)))
+    trees = corpus(108, 400, 1, 60, 3, treegen.OPS + treegen.CLS_BI)
+    trees += ["ln c-0x1p+0", "/ c0x1p+0 c0x0p+0", "+ x0 / c0x0p+0 c-0x0p+0", "* x1 sin exp c0x1.9p+9",
+              "sqrt - c0x1p+0 c0x1p+1", "max x0 < c0x1p+0 c0x1p+1", "exp sqr c0x1p+3", "cos * c0x1p+40 c0x1.8p+2",
+              "- c0x1p-1074 * x2 c0x1p+0", "c0x1p+0", "x1"]
+    arity = {t: 2 for t in "+ - * / < > == != min max".split()}
+    arity.update({t: 1 for t in "sin cos ln exp sqrt sqr".split()})
+    for t in trees:
+        g = rrc._fold(t)
+        toks = g.split()
+        for i, tok in enumerate(toks):
+            a = arity.get(tok, 0)
+            assert a == 0 or not all(k not in arity and k[0] == "c" for k in toks[i + 1:i + 1 + a]), (t, g)
+        # the oracle reads finite constants only
+        g = " ".join({"cinf": "/ c0x1p+0 c0x0p+0", "c-inf": "/ c-0x1p+0 c0x0p+0"}.get(k, "ln c-0x1p+0" if "nan" in k else k)
+                     for k in toks)
+        u, v = od.eval(t), od.eval(g)
+        assert np.all((u.view(np.uint64) == v.view(np.uint64)) | (np.isnan(u) & np.isnan(v))), (t, g)
+    assert rrc._fold("+ x0 * x1 c0x1p+1") == "+ x0 * x1 c0x1p+1"
+    assert rrc._fold("sin + c0x1p+0 c0x1p+1").startswith("c")
+
+
 def test_stack_depth_is_logarithmic():
     # a perfectly balanced tree of 2^8 leaves needs 7 pushes with Sethi-Ullman ordering
     def bal(d):
