@@ -237,6 +237,11 @@ int rr_fitness_batch_noalloc(rr_ctx* ctx, int32_t handle, const rr_batch* batch,
 int rr_predict(rr_ctx* ctx, int32_t handle, const uint32_t* code, int32_t len, const double* consts,
                int32_t n_consts, double* out);
 
+/* The same values for rows that are not a resident dataset: X_rm holds n x d
+ * doubles, row-major, in host memory; out[n].  Nothing is kept of X_rm. */
+int rr_predict_rows(rr_ctx* ctx, const double* X_rm, int64_t n, int32_t d, const uint32_t* code, int32_t len,
+                    const double* consts, int32_t n_consts, double* out);
+
 /* FP32 evaluation of one program with a per-sample bound: |out_v[i] - v64[i]|
  * <= out_e[i], where v64 is what rr_predict returns.  out_e[i] = +inf where
  * FP32 cannot vouch for the sample (overflow, a domain edge inside the

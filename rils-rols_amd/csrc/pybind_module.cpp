@@ -399,13 +399,10 @@ PYBIND11_MODULE(rils_rols_cpp, m) {
            [](RilsRols& self, py::array_t<double, py::array::c_style | py::array::forcecast> X, int data_cnt,
               int feat_cnt) {
              py::buffer_info bx = X.request();
-             std::vector<double> out;
-             {
-               py::gil_scoped_release nogil;
-               out = self.predict((const double*)bx.ptr, bx.size, data_cnt, feat_cnt);
-             }
-             py::array_t<double> res(data_cnt);
-             std::copy(out.begin(), out.end(), (double*)res.request().ptr);
+             py::array_t<double> res(std::max(data_cnt, 0));
+             double* out = (double*)res.request().ptr;
+             py::gil_scoped_release nogil;
+             self.predict((const double*)bx.ptr, bx.size, data_cnt, feat_cnt, out);
              return res;
            })
       .def("get_model_string", &RilsRols::get_model_string)

@@ -252,8 +252,9 @@ hipError_t launch_alive_fp64(const int32_t* ustart, const int32_t* users, const 
 hipError_t launch_xnorm_fp64(const double* X, int64_t n, int64_t ldx, int32_t d, double* out, hipStream_t s);
 hipError_t launch_nan0_fp64(const Nan0Launch& L, hipStream_t s);
 hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s);
+// feature j of row i at X[j col + i row]
 hipError_t launch_predict_fp64(const uint32_t* code, int len, const double* K, const double* X, int64_t n,
-                               int64_t ldx, double* out, hipStream_t s);
+                               int64_t col, int64_t row, double* out, hipStream_t s);
 hipError_t launch_fill_f64(double* p, int64_t count, double value, hipStream_t s);
 // out4 = {mean(y), sum((y - mean)^2), sum(y), sum(y^2)}
 hipError_t launch_stats_fp64(const double* y, int64_t n, double* out4, hipStream_t s);

@@ -902,7 +902,7 @@ void RilsRols::local_search_from(const double* Xp, int64_t x_size, const double*
   final_fitness_ = f;
 }
 
-std::vector<double> RilsRols::predict(const double* Xp, int64_t x_size, int data_cnt, int feat_cnt) {
+void RilsRols::predict(const double* Xp, int64_t x_size, int data_cnt, int feat_cnt, double* out) {
   if (x_size != (int64_t)data_cnt * feat_cnt)
     throw std::invalid_argument("Size of X " + std::to_string(x_size) +
                                 " is not the same as the product of data count and feature count " +
@@ -911,22 +911,14 @@ std::vector<double> RilsRols::predict(const double* Xp, int64_t x_size, int data
   if (!gpu_) gpu_ = new GpuSession(backend_, device_, slab_budget_mb_, ctx_options_);
   rr_ctx* ctx = gpu_->be->context();
   if (!ctx) throw std::runtime_error("predict needs a fitness backend with a device context");
-  std::vector<double> fm((size_t)data_cnt * std::max(feat_cnt, 1));
-  for (int i = 0; i < data_cnt; ++i)
-    for (int j = 0; j < feat_cnt; ++j) fm[(size_t)j * data_cnt + i] = Xp[(int64_t)i * feat_cnt + j];
-  std::vector<double> zeros(data_cnt, 0.0), out(data_cnt);
-  int32_t h = -1;
-  rr_check(rr_dataset_upload(ctx, fm.data(), zeros.data(), data_cnt, feat_cnt, &h), "rr_dataset_upload");
   std::vector<uint32_t> code;
   std::vector<double> consts;
   compile(final_solution_, code, consts);
-  const int rc = rr_predict(ctx, h, code.data(), (int32_t)code.size(), consts.data(), (int32_t)consts.size(),
-                            out.data());
-  rr_dataset_free(ctx, h);
-  rr_check(rc, "rr_predict");
+  rr_check(rr_predict_rows(ctx, Xp, data_cnt, feat_cnt, code.data(), (int32_t)code.size(), consts.data(),
+                           (int32_t)consts.size(), out),
+           "rr_predict_rows");
   if (classification_)
-    for (double& v : out) v = v >= 0.5 ? 1.0 : 0.0;
-  return out;
+    for (int i = 0; i < data_cnt; ++i) out[i] = out[i] >= 0.5 ? 1.0 : 0.0;
 }
 
 std::string RilsRols::get_model_string() const {

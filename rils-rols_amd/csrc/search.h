@@ -92,8 +92,8 @@ class RilsRols {
   // caller (and the tests) drive the batched sweep without the main loop.
   void local_search_from(const double* X, int64_t x_size, const double* y, int64_t y_size, int data_cnt,
                          int feat_cnt, const std::string& prefix);
-  // rils_rols_cpp.cpp:730-750
-  std::vector<double> predict(const double* X, int64_t x_size, int data_cnt, int feat_cnt);
+  // rils_rols_cpp.cpp:730-750 (X row-major; out[data_cnt])
+  void predict(const double* X, int64_t x_size, int data_cnt, int feat_cnt, double* out);
 
   std::string get_model_string() const;
   double get_best_time() const { return best_time_; }

@@ -67,6 +67,8 @@ def lib():
         L.rr_predict.argtypes = [vp, ctypes.c_int32, ctypes.POINTER(ctypes.c_uint32), ctypes.c_int32, dp,
                                  ctypes.c_int32, dp]
         fp = ctypes.POINTER(ctypes.c_float)
+        L.rr_predict_rows.argtypes = [vp, dp, ctypes.c_int64, ctypes.c_int32, ctypes.POINTER(ctypes.c_uint32),
+                                      ctypes.c_int32, dp, ctypes.c_int32, dp]
         L.rr_predict_fp32.argtypes = [vp, ctypes.c_int32, ctypes.POINTER(ctypes.c_uint32), ctypes.c_int32, dp,
                                       ctypes.c_int32, fp, fp]
         L.rr_autotune.argtypes = [vp, ctypes.c_int32, ctypes.POINTER(Batch), ctypes.c_int32, ctypes.c_int32,
@@ -340,6 +342,17 @@ class Context:
         code = arrs["code"]
         check(lib().rr_predict(self.p, h, code.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), len(code),
                                _dp(arrs["consts"]), arrs["n_consts"], _dp(out)))
+        return out
+
+    def predict_rows(self, X, prefix):
+        """`prefix` on the rows of X (n x d, host memory), no dataset."""
+        X = np.ascontiguousarray(X, dtype=np.float64)
+        arrs = build_batch([[prefix]])
+        out = np.empty(X.shape[0])
+        code = arrs["code"]
+        check(lib().rr_predict_rows(self.p, _dp(X), X.shape[0], X.shape[1],
+                                    code.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), len(code),
+                                    _dp(arrs["consts"]), arrs["n_consts"], _dp(out)))
         return out
 
     def predict_fp32(self, h, prefix, n):

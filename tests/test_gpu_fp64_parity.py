@@ -54,6 +54,24 @@ def test_elementwise_ops_bitexact(ctx):
     ctx.free(h)
 
 
+# one row; a slot's last row and the first of the next (4 MiB: 524288 rows of
+# one feature, 26176 of 20); several slots; rows wider than a slot
+@pytest.mark.parametrize("n,d", [(1, 1), (65, 3), (524288, 1), (524289, 1), (26176, 20), (26177, 20), (90001, 20),
+                                 (3, 600000)])
+def test_predict_rows_bitexact(ctx, n, d):
+    print("case: predict_rows n=%d d=%d" % (n, d), flush=True)
+    X = np.random.default_rng(n + d).uniform(-4, 4, (n, d))
+    pre = "+ * c0x1.8p+1 sin x0 / exp x%d c0x1.4p+1" % (d - 1)
+    assert same_bits(ctx.predict_rows(X, pre), O.Dataset(X, np.zeros(n)).eval(pre))
+
+
+def test_predict_rows_argument_errors(ctx):
+    for X, pre in [(np.zeros((0, 2)), "x0"), (np.zeros((4, 2)), "x2")]:
+        with pytest.raises(RuntimeError):
+            ctx.predict_rows(X, pre)
+    assert same_bits(ctx.predict_rows(np.zeros((4, 0)), "c0x1p+0"), np.ones(4))
+
+
 def test_dataset_stats_match(ctx):
     X, y = make_data(3, 1000, 3)
     h = ctx.upload(X, y)
