@@ -159,7 +159,7 @@ struct rr_ctx {
   // from and joined back into `stream`
   hipStream_t side64 = nullptr;
   hipEvent_t fork64 = nullptr, join64 = nullptr;
-  DevBuf d_cand, d_prog, d_code, d_K, d_slab, d_order32, d_coefs, d_fit, d_misc, d_pred_e, d_dstab, d_cand_ds;
+  DevBuf d_cand, d_prog, d_code, d_K, d_slab, d_order32, d_fit, d_misc, d_pred_e, d_dstab, d_cand_ds;
   DevBuf d_f64_off, d_f64_ord;   // FP64 slab offsets and launched position -> candidate
   DevBuf d_fac_prog, d_fac_cand, d_fac_item;   // FP64 factor-evaluation work list
   DevBuf d_prog_item, d_norm_part;              // per program: first work item; per work item: chunk sums
@@ -695,7 +695,7 @@ int rr_destroy(rr_ctx* ctx) {
     (void)hipFree(d.X); (void)hipFree(d.y); (void)hipFree(d.X32); (void)hipFree(d.one); (void)hipFree(d.xnorm);
   }
   DevBuf* bufs[] = {&ctx->d_cand, &ctx->d_prog, &ctx->d_code, &ctx->d_K, &ctx->d_slab, &ctx->d_order32,
-                    &ctx->d_coefs, &ctx->d_fit, &ctx->d_misc, &ctx->d_pred_e, &ctx->d_dstab, &ctx->d_cand_ds,
+                    &ctx->d_fit, &ctx->d_misc, &ctx->d_pred_e, &ctx->d_dstab, &ctx->d_cand_ds,
                     &ctx->d_blk_cand, &ctx->d_blk_chunk, &ctx->d_chunk_base, &ctx->d_work, &ctx->d_work_flags,
                     &ctx->d_f64_off, &ctx->d_f64_ord, &ctx->d_dead, &ctx->d_fac_prog, &ctx->d_fac_cand,
                     &ctx->d_fac_item, &ctx->d_prog_item, &ctx->d_norm_part, &ctx->d_info, &ctx->d_pos_item,
@@ -1099,36 +1099,66 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
                        2 * align_up((size_t)(np + 1) * 8) +   // kept-column offsets per program and per unique factor
                        2 * align_up((size_t)(np + 1) * 4) +   // the users of each unique factor
                        align_up((size_t)nc * 8);              // chunk-factor offsets of the chunked QR
-  if (ctx->h2d_pending) {   // the pending call's staged copy still reads the staging buffer
-    RR_HIP(hipEventSynchronize(ctx->h2d_done));
-    ctx->h2d_pending = false;
-  }
-  if (!t_arena && ctx->h_stage.ensure(s_cand + s_prog + s_code + s_K + s_off + s_tab + s_cds + s_chunks + 2 * s_f64) != RR_OK)
-    return RR_E_NOMEM;
+  // results: the fitness, then the coefficients, in one buffer (one copy back).
+  // RAW calls of the plain FP64 form: the scoring kernel writes the fitness,
+  // 32 bytes a candidate, straight into the pinned result buffer.
+  const size_t fb = (size_t)nc * sizeof(rr_fit), cb = mode == RR_MODE_OLS ? (size_t)ncoef * 8 : 0;
+  HostBuf& hres = async ? ctx->h_res[slot] : ctx->h_out;
+  const bool pinned = !t_arena && hres.ensure(align_up(fb) + cb) == RR_OK;
+  if (async && !pinned) return RR_E_NOMEM;
+  const bool direct = pinned && mode == RR_MODE_RAW && precision == RR_FP64;
+  if (!direct && ctx->d_fit.ensure(align_up(fb) + std::max<size_t>(cb, 8)) != RR_OK) return RR_E_NOMEM;
+  // A small RAW call: its inputs packed into the scoring launch's argument
+  // instead of staged (rr::ScorePack)
+  rr::ScorePack pack;
+  auto pack8 = [](size_t bytes) { return (bytes + 7) & ~size_t(7); };
+  const bool packed = direct && !ctx->use_graph &&
+                      pack8((size_t)(nc + 1) * 4) * 2 + pack8((size_t)(np + 1) * 4) + pack8((size_t)ncode * 4) +
+                              (size_t)std::max(b->n_consts, 1) * 8 + table.size() * sizeof(rr::DsDesc) +
+                              (handles ? pack8((size_t)nc * 4) : 0) <= sizeof pack.words;
+  size_t po = 0;
+  auto to_pack = [&](const void* src, size_t bytes) {
+    const int32_t at = (int32_t)po;
+    if (bytes > 0) memcpy((char*)pack.words + po, src, bytes);
+    po += pack8(bytes);
+    return at;
+  };
+  static const double zero = 0.0;   // a batch without constants: one zero, never read
+  const double* const kp = b->n_consts > 0 ? b->consts : &zero;
+  const size_t kb = (size_t)std::max(b->n_consts, 1) * 8;
   size_t so = 0;
-  if ((rc = upload(ctx, ctx->d_cand, b->cand_start, (size_t)(nc + 1) * 4, so))) return rc;
-  so += s_cand;
-  if ((rc = upload(ctx, ctx->d_prog, b->prog_start, (size_t)(np + 1) * 4, so))) return rc;
-  so += s_prog;
-  if (ncode > 0) { if ((rc = upload(ctx, ctx->d_code, b->code, (size_t)ncode * 4, so))) return rc; }
-  else if (ctx->d_code.ensure(4) != RR_OK) return RR_E_NOMEM;
-  so += s_code;
-  {
-    static const double zero = 0.0;   // a batch without constants: one zero, never read
-    const double* kp = b->n_consts > 0 ? b->consts : &zero;
-    if ((rc = upload(ctx, ctx->d_K, kp, (size_t)std::max(b->n_consts, 1) * 8, so))) return rc;
-  }
-  so += s_K;
-  if ((rc = upload(ctx, ctx->d_dstab, table.data(), table.size() * sizeof(rr::DsDesc), so))) return rc;
-  so += s_tab;
   const int32_t* dcds = nullptr;
-  if (handles) {
-    if ((rc = upload(ctx, ctx->d_cand_ds, cand_ds.data(), (size_t)nc * 4, so))) return rc;
-    dcds = (const int32_t*)ctx->d_cand_ds.p;
+  if (packed) {
+    pack.cand_start = to_pack(b->cand_start, (size_t)(nc + 1) * 4);
+    pack.prog_start = to_pack(b->prog_start, (size_t)(np + 1) * 4);
+    pack.code = to_pack(b->code, (size_t)ncode * 4);
+    pack.K = to_pack(kp, kb);
+    pack.ds = to_pack(table.data(), table.size() * sizeof(rr::DsDesc));
+    pack.cand_ds = handles ? to_pack(cand_ds.data(), (size_t)nc * 4) : -1;
+  } else {
+    if (ctx->h2d_pending) {   // the pending call's staged copy still reads the staging buffer
+      RR_HIP(hipEventSynchronize(ctx->h2d_done));
+      ctx->h2d_pending = false;
+    }
+    if (!t_arena && ctx->h_stage.ensure(s_cand + s_prog + s_code + s_K + s_off + s_tab + s_cds + s_chunks + 2 * s_f64) != RR_OK)
+      return RR_E_NOMEM;
+    if ((rc = upload(ctx, ctx->d_cand, b->cand_start, (size_t)(nc + 1) * 4, so))) return rc;
+    so += s_cand;
+    if ((rc = upload(ctx, ctx->d_prog, b->prog_start, (size_t)(np + 1) * 4, so))) return rc;
+    so += s_prog;
+    if (ncode > 0) { if ((rc = upload(ctx, ctx->d_code, b->code, (size_t)ncode * 4, so))) return rc; }
+    else if (ctx->d_code.ensure(4) != RR_OK) return RR_E_NOMEM;
+    so += s_code;
+    if ((rc = upload(ctx, ctx->d_K, kp, kb, so))) return rc;
+    so += s_K;
+    if ((rc = upload(ctx, ctx->d_dstab, table.data(), table.size() * sizeof(rr::DsDesc), so))) return rc;
+    so += s_tab;
+    if (handles) {
+      if ((rc = upload(ctx, ctx->d_cand_ds, cand_ds.data(), (size_t)nc * 4, so))) return rc;
+      dcds = (const int32_t*)ctx->d_cand_ds.p;
+    }
+    so += s_cds;
   }
-  so += s_cds;
-  if (ctx->d_fit.ensure((size_t)nc * sizeof(rr_fit)) != RR_OK) return RR_E_NOMEM;
-  if (ctx->d_coefs.ensure((size_t)std::max<int64_t>(ncoef, 1) * 8) != RR_OK) return RR_E_NOMEM;
   const int32_t* ddead = nullptr;   // OLS mode: written by the pre-pass for every candidate
   if (mode == RR_MODE_OLS) {
     if (ctx->d_dead.ensure((size_t)std::max(nc, 1) * 4) != RR_OK) return RR_E_NOMEM;
@@ -1141,8 +1171,8 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
   const uint32_t* dcode = (const uint32_t*)ctx->d_code.p;
   const double* dK = (const double*)ctx->d_K.p;
   const rr::DsDesc* dtab = (const rr::DsDesc*)ctx->d_dstab.p;
-  rr_fit* dfit = (rr_fit*)ctx->d_fit.p;
-  double* dcoef = (double*)ctx->d_coefs.p;
+  rr_fit* dfit = (rr_fit*)(direct ? hres.p : ctx->d_fit.p);
+  double* dcoef = direct ? nullptr : (double*)((char*)ctx->d_fit.p + align_up(fb));
 
   // FP32: order, chunk map and workspace
   rr::Fp32Launch L32{};
@@ -1686,7 +1716,12 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     }
     if (it > INT32_MAX) return fail(RR_E_LIMIT, "too many scoring work items in one launch");
     pos_item[nc] = (int32_t)it;
-    if ((rc = upload(ctx, ctx->d_pos_item, pos_item.data(), pos_item.size() * 4, so64))) return rc;
+    if (packed) {
+      pack.pos_item = to_pack(pos_item.data(), pos_item.size() * 4);
+      raw64.pack = &pack;
+    } else if ((rc = upload(ctx, ctx->d_pos_item, pos_item.data(), pos_item.size() * 4, so64))) {
+      return rc;
+    }
     if (ctx->d_score_part.ensure((size_t)std::max<int64_t>(it, 1) * 8) != RR_OK) return RR_E_NOMEM;
     raw64.cand_start = dc; raw64.prog_start = dp; raw64.code = dcode; raw64.K = dK; raw64.ds = dtab;
     raw64.cand_ds = dcds; raw64.prog_kept = nullptr; raw64.order = nullptr; raw64.dead = nullptr; raw64.info = nullptr;
@@ -1701,7 +1736,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
   ctx->ev_used = 0;
   const clk::time_point t_launch = clk::now();
   if ((rc = flush_uploads(ctx))) return rc;
-  if (async) {   // every input of the plain FP64 form is staged by now
+  if (async && !packed) {   // every input of the plain FP64 form is staged by now
     RR_HIP(hipEventRecord(ctx->h2d_done, ctx->stream));
     ctx->h2d_pending = true;
   }
@@ -1765,12 +1800,10 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
   // results: through the pinned buffer h_out (no-alloc calls: straight into
   // the caller's arrays, no host allocation); a pipelined call's through its
   // slot's buffer, completed by wait_oldest
-  const size_t fb = (size_t)nc * sizeof(rr_fit), cb = mode == RR_MODE_OLS ? (size_t)ncoef * 8 : 0;
+  char* const ho = pinned ? (char*)hres.p : nullptr;
+  if (pinned && !direct)
+    RR_HIP(hipMemcpyAsync(ho, dfit, cb ? align_up(fb) + cb : fb, hipMemcpyDeviceToHost, ctx->stream));
   if (async) {
-    if (ctx->h_res[slot].ensure(align_up(fb) + cb) != RR_OK) return RR_E_NOMEM;
-    char* ho = (char*)ctx->h_res[slot].p;
-    RR_HIP(hipMemcpyAsync(ho, dfit, fb, hipMemcpyDeviceToHost, ctx->stream));
-    if (cb) RR_HIP(hipMemcpyAsync(ho + align_up(fb), dcoef, cb, hipMemcpyDeviceToHost, ctx->stream));
     RR_HIP(hipEventRecord(ctx->pdone[slot], ctx->stream));
     rr_ctx::Pending& P = ctx->pend[slot];
     P.fit_out = fit_out; P.coefs_out = coefs_out; P.fb = fb; P.cb = cb; P.ran = false; P.ms = 0.0;
@@ -1780,10 +1813,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     ctx->phase_ms[RR_PHASE_HOST_PLAN] = ms_since(t_checked, t_launch);
     return RR_OK;
   }
-  if (!t_arena && ctx->h_out.ensure(align_up(fb) + cb) == RR_OK) {
-    char* ho = (char*)ctx->h_out.p;
-    RR_HIP(hipMemcpyAsync(ho, dfit, fb, hipMemcpyDeviceToHost, ctx->stream));
-    if (cb) RR_HIP(hipMemcpyAsync(ho + align_up(fb), dcoef, cb, hipMemcpyDeviceToHost, ctx->stream));
+  if (pinned) {
     RR_HIP(hipStreamSynchronize(ctx->stream));
     memcpy(fit_out, ho, fb);
     if (cb) memcpy(coefs_out, ho + align_up(fb), cb);
@@ -1872,7 +1902,7 @@ int rr_fitness_batch_noalloc(rr_ctx* ctx, int32_t handle, const rr_batch* b, int
   // The call runs with every work buffer carved from the scratch array; the
   // context's own buffers are set aside and put back afterwards, untouched.
   DevBuf* bufs[] = {&ctx->d_cand, &ctx->d_prog, &ctx->d_code, &ctx->d_K, &ctx->d_slab, &ctx->d_order32,
-                    &ctx->d_coefs, &ctx->d_fit, &ctx->d_misc, &ctx->d_pred_e, &ctx->d_dstab, &ctx->d_cand_ds,
+                    &ctx->d_fit, &ctx->d_misc, &ctx->d_pred_e, &ctx->d_dstab, &ctx->d_cand_ds,
                     &ctx->d_blk_cand, &ctx->d_blk_chunk, &ctx->d_chunk_base, &ctx->d_work, &ctx->d_work_flags,
                     &ctx->d_f64_off, &ctx->d_f64_ord, &ctx->d_dead, &ctx->d_fac_prog, &ctx->d_fac_cand,
                     &ctx->d_fac_item, &ctx->d_prog_item, &ctx->d_norm_part, &ctx->d_info, &ctx->d_pos_item,

@@ -163,6 +163,18 @@ __host__ __device__ constexpr int ts_block(int nc) { return nc <= 7 ? 256 : 512;
 // (prog_kept), for the candidates whose info is >= 0 -- and then per position
 // the chunk sums in order into the fitness.  Position p owns work items
 // pos_item[p] .. pos_item[p+1]-1 (items_per_pos > 0: p * items_per_pos ..).
+//
+// ScorePack: the inputs of a small RAW call, at byte offsets of its words, as
+// part of the kernel's argument: no staged copy before the kernel.  A staged
+// copy is a kernel of its own (5 us and a dependency of the scoring), so a
+// call of one tree on 150 rows takes 32.4 us with two copies and 21.6 us with none; the
+// limit keeps the argument well inside the 4 KiB a launch can pass, room for
+// about a dozen trees of 20 nodes.
+constexpr int SCORE_PACK_BYTES = 3072;
+struct ScorePack {
+  int32_t cand_start, prog_start, code, K, ds, cand_ds, pos_item;   // cand_ds < 0: none
+  uint64_t words[SCORE_PACK_BYTES / 8];
+};
 struct ScoreLaunch {
   const int32_t* cand_start;
   const int32_t* prog_start;
@@ -184,6 +196,9 @@ struct ScoreLaunch {
   int rows, form, depth;     // RAW: as EvalLaunch's
   double* part;              // per work item
   rr_fit* fit;
+  // RAW, a small call: the input arrays packed in host memory at multiples of
+  // 8 bytes and passed with the launch (the pointers above are unused then)
+  const ScorePack* pack;
 };
 
 // Factor-0 pre-pass of the OLS form: one workgroup per candidate evaluates

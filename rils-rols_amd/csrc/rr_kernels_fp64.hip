@@ -1454,9 +1454,7 @@ __device__ inline void score_finish(const ScoreArgs& a, double s, double (&red)[
 // nodes on 50021 rows takes 713 us with the operand stack in LDS, 840 us with
 // it in registers and the transcendentals called.
 template <int R, int FORM>
-__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_raw(ScoreArgs a) {
-  __shared__ double red[EV_THREADS / WAVE];
-  extern __shared__ double sc_stk[];   // FORM 1: the operand stack
+__device__ inline void score_raw(const ScoreArgs& a, double (&red)[EV_THREADS / WAVE], double* sc_stk) {
   const int item = (int)blockIdx.x;
   const int pos = a.items_per_pos > 0 ? item / a.items_per_pos : score_pos(a, item);
   const int cand = a.order ? a.order[pos] : pos;
@@ -1482,6 +1480,40 @@ __global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_raw(S
     }
   }
   score_finish(a, s, red, item, D, cand, 0);
+}
+template <int R, int FORM>
+__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_raw(ScoreArgs a) {
+  __shared__ double red[EV_THREADS / WAVE];
+  extern __shared__ double sc_stk[];   // FORM 1: the operand stack
+  score_raw<R, FORM>(a, red, sc_stk);
+}
+
+// A RAW call whose inputs are part of the launch's argument (ScorePack), read
+// where the argument is: through the kernel argument segment, so the words
+// are not copied to private memory first.
+struct ScorePackArgs {
+  ScoreArgs a;
+  ScorePack p;
+};
+__device__ inline ScoreArgs unpack_args() {
+  typedef const __attribute__((address_space(4))) ScorePackArgs* argp;
+  const argp g = (argp)__builtin_amdgcn_kernarg_segment_ptr();
+  const char* const w = (const char*)&g->p.words[0];
+  ScoreArgs a = *(const ScoreArgs*)&g->a;
+  a.cand_start = (const int32_t*)(w + g->p.cand_start);
+  a.prog_start = (const int32_t*)(w + g->p.prog_start);
+  a.code = (const uint32_t*)(w + g->p.code);
+  a.K = (const double*)(w + g->p.K);
+  a.ds = (const DsDesc*)(w + g->p.ds);
+  a.cand_ds = g->p.cand_ds < 0 ? nullptr : (const int32_t*)(w + g->p.cand_ds);
+  a.pos_item = (const int32_t*)(w + g->p.pos_item);
+  return a;
+}
+template <int R, int FORM>
+__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_raw_pack(ScorePackArgs) {
+  __shared__ double red[EV_THREADS / WAVE];
+  extern __shared__ double sc_stk[];   // FORM 1: the operand stack
+  score_raw<R, FORM>(unpack_args(), red, sc_stk);
 }
 
 // The OLS tree's prediction from the coefficients and the factor columns, with
@@ -1624,7 +1656,7 @@ __global__ __launch_bounds__(EV_THREADS, 6) void k_score_ols(ScoreArgs a) {
 // One thread per launched position: the chunk sums in chunk order, then the
 // fitness (rils_rols_cpp.cpp:520-541).
 template <bool RAW>
-__global__ __launch_bounds__(256) void k_fit_fp64(ScoreArgs a) {
+__device__ inline void fit_pos(const ScoreArgs& a) {
   const int pos = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (pos >= a.n_pos) return;
   const int cand = a.order ? a.order[pos] : pos;
@@ -1643,6 +1675,11 @@ __global__ __launch_bounds__(256) void k_fit_fp64(ScoreArgs a) {
   ordered_sums<1>(a.part + first, 1, nch, &ssr);
   write_fit(a.fit + cand, ssr, D.sst, D.n, rank, steps);
 }
+template <bool RAW>
+__global__ __launch_bounds__(256) void k_fit_fp64(ScoreArgs a) {
+  fit_pos<RAW>(a);
+}
+__global__ __launch_bounds__(256) void k_fit_raw_pack(ScorePackArgs) { fit_pos<true>(unpack_args()); }
 
 // node::evaluate_all over all samples; many waves, any order (no reduction)
 // One program over n rows; feature j of row i at X[j col + i row]: a dataset's
@@ -2304,6 +2341,17 @@ hipError_t launch_nan0_fp64(const Nan0Launch& L, hipStream_t s) {
   return hipGetLastError();
 }
 
+// the RAW kernel of the launch's rows and form
+#define RR_RAW_FORMS                          \
+  if (L.form == 1 && stk <= EVAL_STACK_MAX) { \
+    if (L.rows == 1) RR_RAW(1, 1, stk);       \
+    else if (L.rows == 4) RR_RAW(4, 1, stk);  \
+    else RR_RAW(2, 1, stk);                   \
+  } else {                                    \
+    if (L.rows == 1) RR_RAW(1, 0, 0);         \
+    else if (L.rows == 4) RR_RAW(4, 0, 0);    \
+    else RR_RAW(2, 0, 0);                     \
+  }
 hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {
   if (L.n_pos <= 0) return hipSuccess;
   // OLS: more chunks a workgroup once the launch is large, to spread a
@@ -2318,15 +2366,17 @@ hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {
   if (L.raw) {
     const dim3 grid((unsigned)L.n_items);
     const size_t stk = eval_stack(L.depth, L.rows);
-    if (L.form == 1 && stk <= EVAL_STACK_MAX) {
-      if (L.rows == 1) hipLaunchKernelGGL((k_score_raw<1, 1>), grid, block, stk, s, a);
-      else if (L.rows == 4) hipLaunchKernelGGL((k_score_raw<4, 1>), grid, block, stk, s, a);
-      else hipLaunchKernelGGL((k_score_raw<2, 1>), grid, block, stk, s, a);
-    } else {
-      if (L.rows == 1) hipLaunchKernelGGL((k_score_raw<1, 0>), grid, block, 0, s, a);
-      else if (L.rows == 4) hipLaunchKernelGGL((k_score_raw<4, 0>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((k_score_raw<2, 0>), grid, block, 0, s, a);
+    if (L.pack) {
+      const ScorePackArgs pa{a, *L.pack};
+#define RR_RAW(R, F, STK) hipLaunchKernelGGL((k_score_raw_pack<R, F>), grid, block, STK, s, pa)
+      RR_RAW_FORMS
+#undef RR_RAW
+      if (L.items_per_pos != 1) hipLaunchKernelGGL(k_fit_raw_pack, fgrid, dim3(POS_THREADS), 0, s, pa);
+      return hipGetLastError();
     }
+#define RR_RAW(R, F, STK) hipLaunchKernelGGL((k_score_raw<R, F>), grid, block, STK, s, a)
+    RR_RAW_FORMS
+#undef RR_RAW
   } else {
     const int64_t blocks = L.items_per_pos > 0 ? (int64_t)L.n_pos * ((L.items_per_pos + span - 1) / span) : L.n_items;
     hipLaunchKernelGGL(k_score_ols, dim3((unsigned)blocks), block, 0, s, a);
@@ -2337,6 +2387,7 @@ hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {
   }
   return hipGetLastError();
 }
+#undef RR_RAW_FORMS
 
 hipError_t launch_predict_fp64(const uint32_t* code, int len, const double* K, const double* X, int64_t n,
                                int64_t col, int64_t row, double* out, hipStream_t s) {

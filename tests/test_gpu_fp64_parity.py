@@ -658,3 +658,37 @@ def test_raw_eval_forms_bitexact(ctx, form, rows):
         ctx.set_option("fp64_eval_rows", 2)
         ctx.set_option("fp64_eval_form", 1)
     ctx.free(h)
+
+
+@pytest.mark.parametrize("sizes", [(1, 64), (150, 150), (4096, 4097), (9000, 33)])
+def test_small_raw_batches_bitexact(ctx, sizes):
+    """Raw calls of 1 to 60 trees: the smallest go out with their inputs in
+    the launch's argument, the others staged; synchronous, pipelined and over
+    two datasets, with one chunk of rows and several."""
+    print("case: small raw batches n=%s" % (sizes,), flush=True)
+    data = [make_data(90 + i, n, 3) for i, n in enumerate(sizes)]
+    hs = [ctx.upload(X, y) for X, y in data]
+    ods = [O.Dataset(X, y) for X, y in data]
+    trees = treegen.random_trees(91, 60, 1, 40, 3)
+    want = [[od.score(t)[:2] for t in trees] for od in ods]
+
+    def check(fit, expected):
+        for f, (e0, e1) in zip(fit, expected):
+            assert same_bits([f["e0"], f["e1"]], [e0, e1])
+    for count in (1, 2, 5, 9, 10, 11, 12, 13, 14, 15, 16, 20, 30, 60):
+        arrs = capi.build_batch([[t] for t in trees[:count]])
+        check(ctx.fitness(hs[0], arrs, mode="raw")[1], want[0])
+        which = [i % 2 for i in range(count)]
+        _, fit = ctx.fitness(None, arrs, mode="raw", handles=[hs[w] for w in which])
+        check(fit, [want[w][i] for i, w in enumerate(which)])
+        first = ctx.submit(hs[1], arrs, mode="raw")
+        second = ctx.submit(hs[0], capi.build_batch([[t] for t in trees[::-1]]), mode="raw")
+        ctx.wait()
+        third = ctx.submit(hs[0], arrs, mode="raw")
+        check(first()[1], want[1])
+        ctx.wait()
+        check(second()[1], want[0][::-1])
+        ctx.wait()
+        check(third()[1], want[0])
+    for h in hs:
+        ctx.free(h)
