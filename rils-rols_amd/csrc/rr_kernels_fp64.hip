@@ -1195,8 +1195,13 @@ static_assert(EVAL_CHUNK_ROWS == rrm::NORM_CHUNK, "evaluation work items are the
 // called; eight waves per SIMD (at two rows per thread the interpreter then
 // fits in 64 VGPRs without new spills).  FORM 1: eval_lds_f64, the operand
 // stack in dynamic LDS (the launch's deepest program x R x EV_THREADS
-// doubles) and the transcendentals inlined.
-constexpr int eval_waves(int rows, int form) { return form == 0 ? 8 : rows <= 2 ? 6 : 4; }
+// doubles) and the transcendentals inlined, six waves per SIMD.  An
+// instruction's fixed part (decode, branches, the operand's latency) serves R
+// rows; at four rows the registers still allow six waves.  Kernel time of 900
+// raw trees on 50021 rows, of the 4096-tree batch on 1e5 rows: 919, 1816 us
+// at one row, 554, 1460 at two, 462, 1425 at four and five waves, 428, 1380
+// at four and six, 430, 1545 at eight rows and four waves.
+constexpr int eval_waves(int, int form) { return form == 0 ? 8 : 6; }
 template <int R, int FORM>
 __global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_eval_fp64(EvalArgs a) {
   static_assert(EV_THREADS == rrm::NORM_PARTIALS, "one thread per partial of the chunked order");
@@ -1450,9 +1455,10 @@ __device__ inline void score_finish(const ScoreArgs& a, double s, double (&red)[
 
 // RAW: one workgroup per work item, the candidate's one program over the chunk.
 // FORM as in k_eval_fp64, whose interpreters and register budgets these are.
-// Bound by the evaluation's instruction issue: a call of 900 trees of about 20
-// nodes on 50021 rows takes 713 us with the operand stack in LDS, 840 us with
-// it in registers and the transcendentals called.
+// Bound by the interpreter's latencies and its instruction issue (58% busy): a
+// call of 900 trees of about 20 nodes on 50021 rows takes 475 us with the
+// operand stack in LDS and four rows a thread, 611 with two rows, and took 840
+// with the stack in registers and the transcendentals called.
 template <int R, int FORM>
 __device__ inline void score_raw(const ScoreArgs& a, double (&red)[EV_THREADS / WAVE], double* sc_stk) {
   const int item = (int)blockIdx.x;
