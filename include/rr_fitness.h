@@ -263,7 +263,8 @@ int rr_predict_fp32(rr_ctx* ctx, int32_t handle, const uint32_t* code, int32_t l
  * 512; default 4096: a candidate's samples are split into chunks that run as
  * independent workgroups, and the chunk sums are added in chunk order),
  * "fp32_streams" (1: the FP32 factor-count buckets run on concurrent streams;
- * default 0, back to back on the context's stream), "host_threads" (host
+ * 0: back to back on the context's stream; 2, the default: concurrently in
+ * calls large enough to gain by it; same bits), "host_threads" (host
  * threads a call may use to check a large batch, 1..64; default 4),
  * "phase_timing" (1: record rr_last_phase_ms; default 0), "graph" (1: the
  * plain FP64 form's launches of a call are captured into a HIP graph and

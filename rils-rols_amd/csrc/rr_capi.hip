@@ -195,7 +195,7 @@ struct rr_ctx {
   int64_t fp64_eval_form = 1;    // the factor interpreter: 0 stack in registers, 1 stack in LDS
   int64_t fp32_rows = 2;
   int64_t fp32_chunk_rows = 4096;
-  int64_t fp32_streams = 0;   // 1: bucket kernels on concurrent side streams
+  int64_t fp32_streams = 2;   // bucket kernels on concurrent side streams: 0 never, 1 always, 2 by the call's size
   int64_t host_threads = 4;   // host threads for checking a large batch
   void* scratch = nullptr;    // device address of this device's scratch array
   double last_ms = 0.0;
@@ -634,6 +634,13 @@ int flush_uploads(rr_ctx* ctx) {
   ctx->up_hi = 0;
   return RR_OK;
 }
+
+// fp32_streams 2: the fewest candidates whose buckets run beside each other.
+// A checked call of 64 random trees takes 300 us one after the other and 308
+// beside each other at 9000 rows (307, 314 at 30000; 264, 265 at 3000), of
+// 256 trees 745 and 539 us (798, 581; 613, 455), of 1024 on 1e5 rows 1294 and
+// 1111 us.
+constexpr int32_t FP32_SIDE_CANDS = 128;
 
 size_t align_up(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -1083,9 +1090,24 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       order = list32;
       counts[0] = n32;
     } else {
+      // longest evaluations first within a bucket (counting sort by cost), so
+      // that none of them starts last and ends the bucket alone
+      std::vector<int32_t> lpt(n32);
+      {
+        constexpr int NB = 4096;
+        std::vector<int32_t> cnt(NB + 1, 0);
+        auto key = [&](int32_t c) {
+          int64_t w = 0;
+          for (int32_t p = b->cand_start[c]; p < b->cand_start[c + 1]; ++p) w += pcost[p];
+          return (int)(NB - 1 - std::min<int64_t>(w, NB - 1));
+        };
+        for (int32_t c : list32) ++cnt[key(c)];
+        for (int i = 0, acc = 0; i <= NB; ++i) { const int32_t t = cnt[i]; cnt[i] = acc; acc += t; }
+        for (int32_t c : list32) lpt[cnt[key(c)]++] = c;
+      }
       std::vector<int8_t> bucket(n32);
       for (int32_t q = 0; q < n32; ++q) {
-        const int32_t c = list32[q];
+        const int32_t c = lpt[q];
         const int nfc = b->cand_start[c + 1] - b->cand_start[c];
         int kb = 0;
         while (kb < rr::FP32_BUCKETS - 1 && nfc > rr::FP32_BUCKET_FACTORS[kb]) ++kb;
@@ -1094,7 +1116,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       }
       int start[rr::FP32_BUCKETS];
       for (int kb = 0, acc = 0; kb < rr::FP32_BUCKETS; ++kb) { start[kb] = acc; acc += counts[kb]; }
-      for (int32_t q = 0; q < n32; ++q) order[start[bucket[q]]++] = list32[q];
+      for (int32_t q = 0; q < n32; ++q) order[start[bucket[q]]++] = lpt[q];
     }
     chunk_base.assign(nc, 0);
     for (int kb = 0, q = 0; kb < rr::FP32_BUCKETS; ++kb) {
@@ -1664,27 +1686,30 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     return RR_OK;
   };
 
-  // FP32 launches on the context's stream (bucket kernels back to back, or
-  // with option fp32_streams bucket 0 there and the others on side streams)
+  // FP32 launches on the context's stream: the bucket kernels back to back,
+  // or beside each other, bucket 0 there and the others on side streams.  A
+  // bucket's kernel is a few long-running workgroups per compute unit with a
+  // tail of its own, so together they fill the chip better.
   auto fp32_run = [&]() -> int {
     if (n32 == 0) return RR_OK;
     const int pm = begin_phase(ctx, RR_PHASE_FP32, ctx->stream);
-    const bool side = ctx->fp32_streams != 0 && mode == RR_MODE_OLS;
+    const bool on = mode == RR_MODE_OLS &&
+                    (ctx->fp32_streams == 1 || (ctx->fp32_streams == 2 && n32 >= FP32_SIDE_CANDS));
     hipStream_t st[rr::FP32_BUCKETS];
-    st[0] = ctx->stream;
-    for (int i = 0; side && i < rr::FP32_BUCKETS - 1; ++i)
-      if ((rc = make_side(&ctx->side[i]))) return rc;
-    for (int i = 1; i < rr::FP32_BUCKETS; ++i) st[i] = side ? ctx->side[i - 1] : ctx->stream;
-    if (side) {
-      RR_HIP(hipEventRecord(ctx->fork, ctx->stream));
-      for (int i = 0; i < rr::FP32_BUCKETS - 1; ++i) RR_HIP(hipStreamWaitEvent(ctx->side[i], ctx->fork, 0));
+    for (hipStream_t& q : st) q = ctx->stream;
+    for (int i = 1; on && i < rr::FP32_BUCKETS; ++i) {
+      if (counts[i] == 0) continue;
+      if ((rc = make_side(&ctx->side[i - 1]))) return rc;
+      st[i] = ctx->side[i - 1];
     }
+    if (on) RR_HIP(hipEventRecord(ctx->fork, ctx->stream));
+    for (int i = 1; i < rr::FP32_BUCKETS; ++i)
+      if (st[i] != ctx->stream) RR_HIP(hipStreamWaitEvent(st[i], ctx->fork, 0));
     RR_HIP(rr::launch_fp32(L32, (const int32_t*)ctx->d_order32.p, counts, blocks, st));
-    if (side) {
-      for (int i = 0; i < rr::FP32_BUCKETS - 1; ++i) {
-        RR_HIP(hipEventRecord(ctx->join[i], ctx->side[i]));
-        RR_HIP(hipStreamWaitEvent(ctx->stream, ctx->join[i], 0));
-      }
+    for (int i = 1; i < rr::FP32_BUCKETS; ++i) {
+      if (st[i] == ctx->stream) continue;
+      RR_HIP(hipEventRecord(ctx->join[i - 1], st[i]));
+      RR_HIP(hipStreamWaitEvent(ctx->stream, ctx->join[i - 1], 0));
     }
     end_phase(ctx, pm, ctx->stream);
     return RR_OK;
@@ -2142,7 +2167,7 @@ int rr_set_option(rr_ctx* ctx, const char* name, int64_t value) {
     if (value != 1 && value != 2) return fail(RR_E_ARG, "fp32_rows must be 1 or 2");
     ctx->fp32_rows = value;
   } else if (s == "fp32_streams") {
-    if (value != 0 && value != 1) return fail(RR_E_ARG, "fp32_streams must be 0 or 1");
+    if (value < 0 || value > 2) return fail(RR_E_ARG, "fp32_streams must be 0, 1 or 2");
     ctx->fp32_streams = value;
   } else if (s == "host_threads") {
     if (value < 1 || value > 64) return fail(RR_E_ARG, "host_threads must be in [1, 64]");

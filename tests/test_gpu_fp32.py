@@ -174,3 +174,27 @@ def test_fp32_random_programs_within_bounds(ctx):
     ctx.free(h)
     print("certified samples %d, worst |v32-v64|/e %.3g" % (total, worst), flush=True)
     assert total > 0
+
+
+@pytest.mark.parametrize("count", [1, 127, 128, 300])
+def test_fp32_streams_same_bits(ctx, count):
+    """The bucket kernels beside each other or one after the other, with and
+    without the FP64 re-scores, below and above the size that switches."""
+    print("case: fp32 streams count=%d" % count, flush=True)
+    import rils_rols_cpp
+    rng = np.random.default_rng(17)
+    X = rng.uniform(-5, 5, (9000, 4))
+    y = np.sin(X[:, 0]) * X[:, 1] + rng.normal(0, 0.01, 9000)
+    facs = [rils_rols_cpp._ols_factors(t) for t in treegen.random_trees(17, 300, 3, 40, 4)]   # up to all buckets
+    arrs = capi.build_batch(facs[:count])
+    h = ctx.upload(X, y)
+    keep = ctx.get_option("fp32_streams")
+    for precision in ("fp32", "fp32c"):
+        got = []
+        for streams in (0, 1, 2):
+            ctx.set_option("fp32_streams", streams)
+            coefs, fit = ctx.fitness(h, arrs, precision=precision)
+            got.append((np.concatenate(coefs).tobytes(), fit.tobytes()))
+        assert got[0] == got[1] == got[2]
+    ctx.set_option("fp32_streams", keep)
+    ctx.free(h)
