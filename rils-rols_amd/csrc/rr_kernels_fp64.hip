@@ -1983,7 +1983,10 @@ __device__ inline void ts_chunk_item(const TsState& st, int64_t r0, int m, doubl
   double v[NC][MR];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    if (c < nc) {   // uniform
+    if (c == kf - 1) {   // uniform: the free term, always the last finite column
+#pragma unroll
+      for (int i = 0; i < MR; ++i) v[c][i] = 1.0;
+    } else if (c < nc) {
       const gcptr src = (gcptr)st.col[c] + r0;
 #pragma unroll
       for (int i = 0; i < MR; ++i) v[c][i] = src[t + THR * i];   // whole chunks exist; rows past m are not used
@@ -2013,8 +2016,9 @@ __device__ inline void ts_chunk_any(const TsState& st, int64_t r0, int m, double
 // The chunk work items of one bucket's live positions (TsList): workgroups
 // take items blockIdx.x, blockIdx.x + gridDim.x, ...
 // Bound by instruction issue (reductions, reflector coefficients, updates) and
-// by the column reads, 9.7 TB/s out of the caches.  A sweep of 800 candidates
-// of 5 to 7 columns with y over 1e6 rows takes 3.46 ms; 8.91 ms with the
+// by the column reads out of the caches.  A sweep of 800 candidates of 5 to 7
+// columns with y over 1e6 rows takes 2.83 ms (3.29 ms with the column of ones
+// read too, whose registers spilled); 8.91 ms with the
 // oracle's 1024 threads as the workgroup (4 rows each), plain butterflies and
 // every thread computing all coefficients: the reductions and the scalar work
 // ran in 16 waves per chunk instead of 4.  At 7500 rows 45 us instead of 98.
