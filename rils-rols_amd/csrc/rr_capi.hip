@@ -505,10 +505,12 @@ bool program_ok(const uint32_t* code, int32_t len, int32_t d, int32_t n_consts, 
 // (rough FP64 instruction units): used only to launch the long evaluations
 // first, so that one of them does not start last and end the launch alone;
 // it changes no result.  prog_hash[p], when asked for, gets the hash of
-// program_ok<true> (equal programs: equal hashes).  threads: host threads it
+// program_ok<true> (equal programs: equal hashes); prog_depth[p] its operand
+// stack's depth.  threads: host threads it
 // may use for a large batch.
 int check_batch(const rr_batch* b, int32_t mode, int32_t d, const int32_t* cand_d, std::vector<int32_t>* prog_cost,
-                std::vector<uint64_t>* prog_hash = nullptr, int threads = 1, int32_t* max_depth = nullptr) {
+                std::vector<uint64_t>* prog_hash = nullptr, int threads = 1, int32_t* max_depth = nullptr,
+                std::vector<uint8_t>* prog_depth = nullptr) {
   if (!b || b->n_cands < 0) return fail(RR_E_ARG, "bad batch");
   if (b->n_cands == 0) return RR_OK;
   if (!b->cand_start || !b->prog_start || (b->n_consts > 0 && !b->consts)) return fail(RR_E_ARG, "null batch array");
@@ -526,6 +528,7 @@ int check_batch(const rr_batch* b, int32_t mode, int32_t d, const int32_t* cand_
     if (b->prog_start[p + 1] < b->prog_start[p]) return fail(RR_E_ARG, "prog_start not monotone");
   if (prog_cost) prog_cost->assign(std::max(n_progs, 1), 0);
   if (prog_hash) prog_hash->resize(std::max(n_progs, 1));
+  if (prog_depth) prog_depth->resize(std::max(n_progs, 1));
   static const double zero = 0.0;   // constant reads of a batch without constants
   const double* K = b->n_consts > 0 ? b->consts : &zero;
   // candidates [c0, c1): the first invalid program, or -1
@@ -539,10 +542,13 @@ int check_batch(const rr_batch* b, int32_t mode, int32_t d, const int32_t* cand_
       for (int32_t p = b->cand_start[c]; p < b->cand_start[c + 1]; ++p) {
         const int32_t len = b->prog_start[p + 1] - b->prog_start[p];
         int64_t w = 0;
+        int32_t dp = 0;
         const bool ok = prog_hash ? program_ok<true>(b->code + b->prog_start[p], len, dc, b->n_consts, K, &w,
-                                                     &(*prog_hash)[p], depth)
+                                                     &(*prog_hash)[p], &dp)
                                   : program_ok<false>(b->code + b->prog_start[p], len, dc, b->n_consts, K, &w, nullptr,
-                                                      depth);
+                                                      &dp);
+        *depth = std::max(*depth, dp);
+        if (prog_depth) (*prog_depth)[p] = (uint8_t)dp;
         if (!ok) { *bad_prog = p; *bad_cand = c; return; }
         if (prog_cost) (*prog_cost)[p] = (int32_t)std::min<int64_t>(w, INT32_MAX);
       }
@@ -1026,6 +1032,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
   }
   std::vector<int32_t> pcost;   // per program: evaluation cost (filled by the check)
   std::vector<uint64_t> phash;  // per program: hash by value (filled by the check, OLS mode)
+  std::vector<uint8_t> pdepth;  // per program: operand stack depth (filled by the check)
   int32_t batch_depth = 0;      // the deepest operand stack of any program (filled by the check)
   {
     std::vector<int32_t> cand_d;
@@ -1034,7 +1041,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       for (int32_t c = 0; c < nc; ++c) cand_d[c] = ctx->ds[uniq[cand_ds[c]]].d;
     }
     if ((rc = check_batch(b, mode, min_d, handles ? cand_d.data() : nullptr, &pcost,
-                          mode == RR_MODE_OLS ? &phash : nullptr, (int)ctx->host_threads, &batch_depth)))
+                          mode == RR_MODE_OLS ? &phash : nullptr, (int)ctx->host_threads, &batch_depth, &pdepth)))
       return rc;
   }
   if (!fit_out) return fail(RR_E_ARG, "null fit_out");
@@ -1484,7 +1491,7 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
       for (int i = 0; i < ch.npair; ++i) {
         const int32_t u = sorted[i], w = ch.p0 + i;
         const int64_t nch = (ds_of(u_cand[u]).n + rr::EVAL_CHUNK_ROWS - 1) / rr::EVAL_CHUNK_ROWS;
-        pprog[w] = u_prog[u];
+        pprog[w] = pdepth[u_prog[u]] > rr::EVAL_LDS_SLOTS ? ~u_prog[u] : u_prog[u];
         pcand[w] = u_cand[u];
         pkept[w] = u_kept[u];
         pitem[w] = (int32_t)items;

@@ -222,12 +222,20 @@ constexpr int NAN0_ROWS = 64;
 // Factor evaluation of the FP64 OLS form into the kept slab columns: one
 // workgroup per (unique factor, chunk of EVAL_CHUNK_ROWS rows).  A unique
 // factor is a program over a dataset that one or more candidates use;
-// factor f is program fac_prog[f] over the dataset of candidate fac_cand[f],
+// factor f is program fac_prog[f] (~fac_prog[f] where negative: a program
+// whose operand stack is deeper than EVAL_LDS_SLOTS) over the dataset of
+// candidate fac_cand[f],
 // kept at slab + fac_kept[f], and owns work items fac_item[f] ..
 // fac_item[f+1]-1, n_items in all.  Work item b also leaves the sums of
 // squares of its chunk in norm_part[2b], norm_part[2b+1].  Factors with
 // alive[f] == 0 (every user candidate settled by the factor-0 pre-pass) are
 // skipped.  Must run before the QR launches over the same candidates.
+// At four rows a thread the LDS holds EVAL_LDS_SLOTS stack slots, 24 KiB, which
+// six workgroups per compute unit fit; the deeper programs (one random tree of
+// 50 nodes in 500) take one row at a time.  Sized for the deepest program of
+// the launch, a batch of 4000 such trees on 1e5 rows took 1455 us of kernels
+// with four programs of depth 4 among them and 1345 without; now 1345.
+constexpr int EVAL_LDS_SLOTS = 3;
 struct EvalLaunch {
   const int32_t* prog_start;
   const uint32_t* code;

@@ -1220,7 +1220,7 @@ __global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_eval_fp64(E
     }
   }
   if (!a.alive[lo]) return;
-  const int cand = a.fac_cand[lo], prog = a.fac_prog[lo];
+  const int cand = a.fac_cand[lo], fp = a.fac_prog[lo], prog = fp < 0 ? ~fp : fp;
   const DsDesc& D = a.ds[a.cand_ds ? a.cand_ds[cand] : 0];
   const uint32_t* code = a.code + a.prog_start[prog];
   const int len = a.prog_start[prog + 1] - a.prog_start[prog];
@@ -1232,19 +1232,28 @@ __global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_eval_fp64(E
   // EV_THREADS * R (which divides 4096) and below n, so every row touched is
   // below ldx.
   double s[2] = {0.0, 0.0};   // rows >= 0, rows >= 1
-  for (int64_t base = r0; base < r1; base += (int64_t)EV_THREADS * R) {
-    const int64_t row0 = base + (int64_t)threadIdx.x;
-    double v[R];
-    if constexpr (FORM == 1) eval_lds_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v, ev_stk);
-    else eval_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v);
+  const auto put = [&](int64_t i, double x) {
+    keep[i] = x;
+    if (i < r1) {
+      s[0] = s[0] + x * x;
+      if (i >= 1) s[1] = s[1] + x * x;
+    }
+  };
+  if (FORM == 1 && R == 4 && fp < 0) {   // a deep operand stack: one row at a time
+    for (int64_t base = r0; base < r1; base += EV_THREADS) {
+      const int64_t row0 = base + (int64_t)threadIdx.x;
+      double v[1];
+      eval_lds_f64<1, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v, ev_stk);
+      put(row0, v[0]);
+    }
+  } else {
+    for (int64_t base = r0; base < r1; base += (int64_t)EV_THREADS * R) {
+      const int64_t row0 = base + (int64_t)threadIdx.x;
+      double v[R];
+      if constexpr (FORM == 1) eval_lds_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v, ev_stk);
+      else eval_f64<R, EV_THREADS>(code, len, a.K, D.X, D.ldx, row0, v);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int64_t i = row0 + (int64_t)EV_THREADS * r;
-      keep[i] = v[r];
-      if (i < r1) {
-        s[0] = s[0] + v[r] * v[r];
-        if (i >= 1) s[1] = s[1] + v[r] * v[r];
-      }
+      for (int r = 0; r < R; ++r) put(row0 + (int64_t)EV_THREADS * r, v[r]);
     }
   }
   s[0] = wave_sum(s[0]);
@@ -2315,7 +2324,9 @@ hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s) {
   EvalArgs a{L.prog_start, L.code,     L.K,        L.ds,       L.cand_ds, L.slab,          L.fac_prog,
              L.fac_cand,   L.fac_item, L.fac_kept, L.alive, L.n_facs,  L.items_per_fac, L.norm_part};
   const dim3 grid((unsigned)L.n_items), block(EV_THREADS);
-  const size_t stk = eval_stack(L.depth, L.rows);
+  // four rows: at most EVAL_LDS_SLOTS slots of four, which are enough for one row of any depth
+  static_assert(4 * EVAL_LDS_SLOTS >= RR_MAX_STACK, "the stack of one row of a deep program");
+  const size_t stk = eval_stack(L.rows == 4 ? std::min(L.depth, EVAL_LDS_SLOTS) : L.depth, L.rows);
   if (L.form == 1 && stk <= EVAL_STACK_MAX) {
     if (L.rows == 1) hipLaunchKernelGGL((k_eval_fp64<1, 1>), grid, block, stk, s, a);
     else if (L.rows == 4) hipLaunchKernelGGL((k_eval_fp64<4, 1>), grid, block, stk, s, a);

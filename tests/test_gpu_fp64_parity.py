@@ -692,3 +692,25 @@ def test_small_raw_batches_bitexact(ctx, sizes):
         check(third()[1], want[0])
     for h in hs:
         ctx.free(h)
+
+
+@pytest.mark.parametrize("n", [513, 4097])
+@pytest.mark.parametrize("levels", [4, 5, 6, 8])
+def test_deep_stacks_at_four_rows_bitexact(ctx, n, levels):
+    """Programs whose operand stack fits the LDS slots of four rows a thread
+    beside programs that take one row at a time."""
+    print("case: deep stacks n=%d levels=%d" % (n, levels), flush=True)
+    rng = np.random.default_rng(levels)
+    X, y = make_data(70 + levels, n, 4)
+    trees = ["* sin %s x1" % _full_tree(rng, L, 4) for L in (1, 2, 3, levels, levels)]
+    od = O.Dataset(X, y)
+    tuned = [od.tune(t) for t in trees]
+    keep = ctx.get_option("fp64_eval_rows")
+    ctx.set_option("fp64_eval_rows", 4)
+    h = ctx.upload(X, y)
+    coefs, fit = ctx.fitness(h, capi.build_batch([tu["factors"] for tu in tuned]), mode="ols")
+    ctx.set_option("fp64_eval_rows", keep)
+    ctx.free(h)
+    for t, tu, c, f in zip(trees, tuned, coefs, fit):
+        assert same_bits(c, tu["coefs"]), (t, c, tu["coefs"])
+        assert same_bits([f["e0"], f["e1"]], [tu["fit"][0], tu["fit"][1]]), (t, f, tu["fit"])
