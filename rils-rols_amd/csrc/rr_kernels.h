@@ -270,16 +270,27 @@ hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s);
 // chunk's chunked QR
 hipError_t launch_alive_fp64(const int32_t* ustart, const int32_t* users, const int32_t* dead, int32_t n,
                              int32_t* alive, const LiveLaunch* live, hipStream_t s);
-// out[2f], out[2f+1]: sums of squares of feature f's column over rows >= 0
-// and rows >= 1 in the chunked order (rrm::chunk_sum)
-hipError_t launch_xnorm_fp64(const double* X, int64_t n, int64_t ldx, int32_t d, double* out, hipStream_t s);
 hipError_t launch_nan0_fp64(const Nan0Launch& L, hipStream_t s);
 hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s);
 // feature j of row i at X[j col + i row]
 hipError_t launch_predict_fp64(const uint32_t* code, int len, const double* K, const double* X, int64_t n,
                                int64_t col, int64_t row, double* out, hipStream_t s);
-hipError_t launch_fill_f64(double* p, int64_t count, double value, hipStream_t s);
-// out4 = {mean(y), sum((y - mean)^2), sum(y), sum(y^2)}
-hipError_t launch_stats_fp64(const double* y, int64_t n, double* out4, hipStream_t s);
+// Dataset upload.  launch_place moves `count` values of the flat input [d
+// columns of n rows | y], from flat index `at` on, to their padded columns
+// (and the FP32 copies); launch_place_stats, after all of them, fills the rows
+// past n and the column of ones and leaves xnorm[2f], xnorm[2f+1], the sums of
+// squares of feature f's column over rows >= 0 and rows >= 1 in the chunked
+// order (rrm::chunk_sum), and out4 = {mean(y), sum((y - mean)^2), sum(y),
+// sum(y^2)}.  part: 2 doubles per feature and chunk of EVAL_CHUNK_ROWS rows.
+struct DsPlace {
+  double* X;
+  float* X32;
+  double* y;
+  double* one;
+  int64_t n, ldx;
+  int d;
+};
+hipError_t launch_place(const double* src, int64_t at, int64_t count, const DsPlace& p, hipStream_t s);
+hipError_t launch_place_stats(const DsPlace& p, double* part, double* xnorm, double* out4, hipStream_t s);
 
 }  // namespace rr

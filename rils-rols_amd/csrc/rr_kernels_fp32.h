@@ -45,7 +45,6 @@ constexpr int FP32_BUCKET_FACTORS[FP32_BUCKETS - 1] = {1, 2, 4, 8};
 // streams).  RAW mode uses order as is and bucket 0's counts, on streams[0].
 hipError_t launch_fp32(const Fp32Launch& L, const int32_t* order, const int* bucket_count, const int* bucket_blocks,
                        const hipStream_t* streams);
-hipError_t launch_to_fp32(const double* src, float* dst, int64_t count, hipStream_t s);
 // FP32 prediction with per-sample bounds (ldx a multiple of 256)
 hipError_t launch_predict_fp32(const uint32_t* code, int len, const double* K, const float* X, int64_t n, int64_t ldx,
                                float* out_v, float* out_e, hipStream_t s);

@@ -187,7 +187,7 @@ __device__ inline VE const_ve(double kd) {
 
 // FP32 evaluation of one program at R samples (rows row0 + 64 r); st[r]
 // receives the row state.  X holds the FP32 copy of the features (tiny
-// nonzero and non-finite entries stored as NaN, see k_to_fp32).
+// nonzero and non-finite entries stored as NaN, see fp32_copy).
 template <int R>
 __device__ inline void eval_f32(const uint32_t* __restrict__ code, int len, const double* __restrict__ K,
                                 const float* __restrict__ X, int64_t ldx, int64_t row0, VE (&acc)[R],
@@ -824,19 +824,6 @@ __global__ __launch_bounds__(256) void k_predict_fp32(const uint32_t* code, int 
   }
 }
 
-// FP32 copy of a column block.  Entries FP32 cannot carry with relative
-// error 2^-24 (non-finite, beyond the FP32 range, nonzero below 2^-100) are
-// stored as NaN, which the evaluator reports as uncertain.
-__global__ void k_to_fp32(const double* src, float* dst, int64_t count) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) {
-    const double x = src[i];
-    const double ax = __builtin_fabs(x);
-    const bool ok = ax == 0.0 || (ax >= 0x1p-100 && ax <= 0x1p127);
-    dst[i] = ok ? (float)x : __builtin_nanf("");
-  }
-}
-
 __global__ void k_needs64(const int32_t* order, int count, const int32_t* cand_start, const int32_t* dead,
                           double* coefs, rr_fit* fit) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
@@ -849,12 +836,6 @@ __global__ void k_needs64(const int32_t* order, int count, const int32_t* cand_s
 }
 
 }  // namespace
-
-hipError_t launch_to_fp32(const double* src, float* dst, int64_t count, hipStream_t s) {
-  if (count <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_to_fp32, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, src, dst, count);
-  return hipGetLastError();
-}
 
 hipError_t launch_predict_fp32(const uint32_t* code, int len, const double* K, const float* X, int64_t n, int64_t ldx,
                                float* out_v, float* out_e, hipStream_t s) {

@@ -1332,35 +1332,68 @@ __global__ __launch_bounds__(ALIVE_THREADS) void k_alive_fp64(const int32_t* ust
   if (threadIdx.x == 0) { T.cnt[b] = n_live; T.cnt[TS_BUCKETS + b] = n_items; }
 }
 
-// Per feature of a dataset, the sums of squares of its column over rows >= 0
-// and rows >= 1 in the chunked order (one workgroup per feature, the chunks
-// in order): the norms the FP64 OLS form uses for a bare-variable factor.
-__global__ __launch_bounds__(EV_THREADS) void k_xnorm_fp64(const double* X, int64_t n, int64_t ldx, double* out) {
-  __shared__ double red[EV_THREADS / WAVE][2];
-  const double* x = X + (int64_t)blockIdx.x * ldx;
-  const int wave = (int)(threadIdx.x / WAVE);
-  double tot0 = 0.0, tot1 = 0.0;
-  for (int64_t r0 = 0; r0 < n; r0 += rrm::NORM_CHUNK) {
-    const int64_t r1 = (r0 + rrm::NORM_CHUNK < n) ? r0 + rrm::NORM_CHUNK : n;
-    double s[2] = {0.0, 0.0};
-    for (int64_t i = r0 + (int64_t)threadIdx.x; i < r1; i += EV_THREADS) {
-      const double v = x[i];
-      s[0] = s[0] + v * v;
-      if (i >= 1) s[1] = s[1] + v * v;
+// ---------------------------------------------------------------- dataset upload
+// The FP32 copy of a feature value.  Values FP32 cannot carry with relative
+// error 2^-24 (non-finite, beyond the FP32 range, nonzero below 2^-100) are
+// stored as NaN, which the FP32 evaluator reports as uncertain.
+__device__ inline float fp32_copy(double x) {
+  const double ax = __builtin_fabs(x);
+  return ax == 0.0 || (ax >= 0x1p-100 && ax <= 0x1p127) ? (float)x : __builtin_nanf("");
+}
+
+// A piece of the flat input [d columns of n rows | y]: its `count` values from
+// flat index `at` on to their places in the padded columns, with the FP32
+// copies of the features.
+__global__ __launch_bounds__(EV_THREADS) void k_place(const double* src, int64_t at, int64_t count, DsPlace p) {
+  for (int64_t i = (int64_t)blockIdx.x * EV_THREADS + threadIdx.x; i < count; i += (int64_t)gridDim.x * EV_THREADS) {
+    const int64_t g = at + i, col = g / p.n, row = g - col * p.n;
+    const double v = src[i];
+    if (col < p.d) {
+      p.X[col * p.ldx + row] = v;
+      p.X32[col * p.ldx + row] = fp32_copy(v);
+    } else {
+      p.y[row] = v;
     }
-    s[0] = wave_sum(s[0]);
-    s[1] = wave_sum(s[1]);
-    if ((threadIdx.x & (WAVE - 1)) == 0) { red[wave][0] = s[0]; red[wave][1] = s[1]; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double t0 = red[0][0], t1 = red[0][1];
-      for (int w = 1; w < EV_THREADS / WAVE; ++w) { t0 = t0 + red[w][0]; t1 = t1 + red[w][1]; }
-      tot0 = (r0 == 0) ? t0 : tot0 + t0;
-      tot1 = (r0 == 0) ? t1 : tot1 + t1;
-    }
-    __syncthreads();   // red is reused by the next chunk
   }
-  if (threadIdx.x == 0) { out[2 * blockIdx.x] = tot0; out[2 * blockIdx.x + 1] = tot1; }
+}
+
+// Block chunk + column x chunks: the chunk's sums of squares of a feature's column
+// over rows >= 0 and rows >= 1 (in the order of rrm::chunk_sum), and zeros in
+// the rows past n.  The block column after the features: y's zeros and the
+// column of ones.
+__global__ __launch_bounds__(EV_THREADS) void k_place_pads(DsPlace p, int chunks, double* part) {
+  __shared__ double red[EV_THREADS / WAVE][2];
+  const int col = (int)blockIdx.x / chunks, chunk = (int)blockIdx.x - col * chunks, cols = p.d > 0 ? p.d : 1;
+  const int64_t r0 = (int64_t)chunk * rrm::NORM_CHUNK;
+  double* const x = col < cols ? p.X + (int64_t)col * p.ldx : p.y;
+  const int64_t n = col < cols && col >= p.d ? 0 : p.n;   // without features the one column is all padding
+  double s[2] = {0.0, 0.0};
+  for (int64_t i = r0 + (int64_t)threadIdx.x; i < r0 + rrm::NORM_CHUNK; i += EV_THREADS) {   // below ldx
+    if (col >= cols) p.one[i] = 1.0;
+    if (i < n) {
+      if (col < cols) {
+        const double v = x[i];
+        s[0] = s[0] + v * v;
+        if (i >= 1) s[1] = s[1] + v * v;
+      }
+    } else {
+      x[i] = 0.0;
+      if (col < cols) p.X32[(int64_t)col * p.ldx + i] = 0.f;
+    }
+  }
+  if (col >= p.d) return;   // uniform
+  s[0] = wave_sum(s[0]);
+  s[1] = wave_sum(s[1]);
+  const int wave = (int)(threadIdx.x / WAVE);
+  if ((threadIdx.x & (WAVE - 1)) == 0) { red[wave][0] = s[0]; red[wave][1] = s[1]; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t0 = red[0][0], t1 = red[0][1];
+    for (int w = 1; w < EV_THREADS / WAVE; ++w) { t0 = t0 + red[w][0]; t1 = t1 + red[w][1]; }
+    double* const o = part + 2 * (int64_t)blockIdx.x;
+    o[0] = t0;
+    o[1] = t1;
+  }
 }
 
 // The factor-0 pre-pass: one workgroup of NAN0_ROWS threads (one wave) per candidate,
@@ -1709,18 +1742,34 @@ __global__ __launch_bounds__(256) void k_predict_fp64(const uint32_t* code, int 
   if (i < n) out[i] = v[0];
 }
 
-// out4: mean of y, sum (y - mean)^2, sum y (canonical sums), sum y^2 (any
-// order: used by the FP32 form only)
-__global__ __launch_bounds__(CP) void k_stats_fp64(const double* y, int64_t n, double* out4) {
+// One workgroup.  Per feature its chunk sums in order (chunks of them each):
+// the norms of a bare-variable factor.  out4: mean of y, sum (y - mean)^2, sum
+// y (canonical sums), sum y^2 (any order: used by the FP32 form only).  A
+// thread's rows are one chain of additions; the loads of eight of them go out
+// together (1e6 rows: 550 us with one at a time, 250 now).
+__global__ __launch_bounds__(CP) void k_stats_fp64(const double* y, int64_t n, const double* part, int64_t chunks,
+                                                   int d, double* xnorm, double* out4) {
   __shared__ double red2[CW][2];
   __shared__ double red1[CW][1];
   const int tid = (int)threadIdx.x;
+  for (int f = tid; f < d; f += CP) ordered_sums<2>(part + 2 * (int64_t)f * chunks, 2, chunks, xnorm + 2 * f);
+  const auto rows = [&](auto add) {   // add(y[i]) for the thread's rows in increasing order
+    int64_t i = tid;
+    for (; i + 7 * CP < n; i += 8 * CP) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = y[i + u * CP];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) add(v[u]);
+    }
+    for (; i < n; i += CP) add(y[i]);
+  };
   double s[2] = {0.0, 0.0};
-  for (int64_t i = tid; i < n; i += CP) { s[0] = s[0] + y[i]; s[1] = __builtin_fma(y[i], y[i], s[1]); }
+  rows([&](double v) { s[0] = s[0] + v; s[1] = __builtin_fma(v, v, s[1]); });
   block_sums<2>(s, red2);
   const double ybar = s[0] / (double)n;
   double q[1] = {0.0};
-  for (int64_t i = tid; i < n; i += CP) q[0] = q[0] + (y[i] - ybar) * (y[i] - ybar);
+  rows([&](double v) { q[0] = q[0] + (v - ybar) * (v - ybar); });
   block_sums<1>(q, red1);
   if (tid == 0) { out4[0] = ybar; out4[1] = q[0]; out4[2] = s[0]; out4[3] = s[1]; }
 }
@@ -2349,9 +2398,19 @@ hipError_t launch_alive_fp64(const int32_t* ustart, const int32_t* users, const 
   return hipGetLastError();
 }
 
-hipError_t launch_xnorm_fp64(const double* X, int64_t n, int64_t ldx, int32_t d, double* out, hipStream_t s) {
-  if (d <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_xnorm_fp64, dim3((unsigned)d), dim3(EV_THREADS), 0, s, X, n, ldx, out);
+hipError_t launch_place(const double* src, int64_t at, int64_t count, const DsPlace& p, hipStream_t s) {
+  if (count <= 0) return hipSuccess;
+  const int64_t blocks = (count + EV_THREADS - 1) / EV_THREADS;
+  hipLaunchKernelGGL(k_place, dim3((unsigned)std::min<int64_t>(blocks, 8192)), dim3(EV_THREADS), 0, s, src, at, count, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_place_stats(const DsPlace& p, double* part, double* xnorm, double* out4, hipStream_t s) {
+  const int64_t chunks = p.ldx / rrm::NORM_CHUNK;
+  const int64_t blocks = chunks * ((int64_t)std::max(p.d, 1) + 1);
+  if (blocks > INT32_MAX) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_place_pads, dim3((unsigned)blocks), dim3(EV_THREADS), 0, s, p, (int)chunks, part);
+  hipLaunchKernelGGL(k_stats_fp64, dim3(1), dim3(CP), 0, s, p.y, p.n, part, chunks, p.d, xnorm, out4);
   return hipGetLastError();
 }
 
@@ -2416,24 +2475,6 @@ hipError_t launch_predict_fp64(const uint32_t* code, int len, const double* K, c
   hipLaunchKernelGGL(k_predict_fp64, dim3((unsigned)blocks), dim3(256), 0, s, code, len, K, X, n, col, row, out);
   return hipGetLastError();
 }
-
-__global__ void k_fill_f64(double* p, int64_t count, double value) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = value;
-}
-
-hipError_t launch_fill_f64(double* p, int64_t count, double value, hipStream_t s) {
-  if (count <= 0) return hipSuccess;
-  const int64_t blocks = (count + 255) / 256;
-  hipLaunchKernelGGL(k_fill_f64, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, p, count, value);
-  return hipGetLastError();
-}
-
-hipError_t launch_stats_fp64(const double* y, int64_t n, double* out4, hipStream_t s) {
-  hipLaunchKernelGGL(k_stats_fp64, dim3(1), dim3(CP), 0, s, y, n, out4);
-  return hipGetLastError();
-}
-
 
 static TsArgs ts_args(const TsLaunch& L, int pos0, int bucket) {
   return TsArgs{L.cand_start, L.ds, L.cand_ds, L.coefs, L.fit, L.dead, L.info, L.order,

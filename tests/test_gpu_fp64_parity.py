@@ -79,6 +79,25 @@ def test_dataset_stats_match(ctx):
     ctx.free(h)
 
 
+# one row; whole and ragged chunks; one slot's worth of values (4 MiB) and one
+# value more; a column across two slots
+@pytest.mark.parametrize("n,d", [(1, 1), (4096, 3), (4097, 3), (262144, 1), (262145, 1), (100001, 11)])
+def test_upload_places_columns_and_statistics(ctx, n, d):
+    print("case: upload n=%d d=%d" % (n, d), flush=True)
+    X, y = make_data(5, n, d)
+    h = ctx.upload(X, y)
+    assert ctx.stats(h) == O.Dataset(X, y).stats()
+    for j in {0, d // 2, d - 1}:
+        assert same_bits(ctx.predict(h, "x%d" % j, n), X[:, j])
+        v, e = ctx.predict_fp32(h, "x%d" % j, n)
+        assert np.array_equal(v, X[:, j].astype(np.float32))
+    od = O.Dataset(X, y)   # y, the ones and the norms of bare factors
+    tu = od.tune("+ x0 x%d" % (d - 1))
+    coefs, fit = ctx.fitness(h, capi.build_batch([tu["factors"]]), mode="ols")
+    assert same_bits(coefs[0], tu["coefs"]) and same_bits([fit[0]["e0"], fit[0]["e1"]], tu["fit"][:2])
+    ctx.free(h)
+
+
 @pytest.mark.parametrize("n,d,seed", [(150, 2, 1), (1000, 5, 2), (4099, 10, 3)])
 def test_raw_fitness_bitexact(ctx, n, d, seed):
     print("case: raw n=%d d=%d seed=%d" % (n, d, seed), flush=True)
