@@ -649,6 +649,14 @@ int flush_uploads(rr_ctx* ctx) {
 // 1111 us.
 constexpr int32_t FP32_SIDE_CANDS = 128;
 
+// A checked call with fewer FP32 chunks scores the candidates that go to FP64
+// up front together with the re-scores: an FP64 launch is a chain of ten
+// dependent kernels, and two of them cost a small call more than the second
+// hides beside the FP32 kernels.  256 trees on 300 rows: 278 us in one launch,
+// 313 in two; 64 on 3000 rows: 284, 318; 256 on 9000: 476, 516; from 500
+// trees on 20000 rows on they are even, or either way by the batch.
+constexpr int64_t FP32_JOIN_CHUNKS = 1024;
+
 size_t align_up(size_t x) { return (x + 255) & ~size_t(255); }
 
 // rr_predict_rows, rr_dataset_upload: bytes of rows per slot.  Bound by the host's copies and the
@@ -1804,8 +1812,11 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     raw64.rows = erows; raw64.form = (int)ctx->fp64_eval_form; raw64.depth = batch_depth;
     raw64.part = (double*)ctx->d_score_part.p; raw64.fit = dfit;
   }
-  if (checked && (rc = make_side(&ctx->side64))) return rc;
-  if (checked && !list64.empty()) { if ((rc = plan64(&list64, 0, plan))) return rc; }
+  // small checked calls: the FP64-bound candidates join the re-scores' launch
+  const bool join64 = checked && total_chunks < FP32_JOIN_CHUNKS;
+  if (checked && !join64 && !list64.empty()) {
+    if ((rc = make_side(&ctx->side64)) || (rc = plan64(&list64, 0, plan))) return rc;
+  }
   // the timed region starts with every input uploaded
   ctx->marks.clear();
   ctx->ev_used = 0;
@@ -1848,13 +1859,14 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     if ((rc = prepass())) return rc;
     if ((rc = fp32_run())) return rc;
   } else {
-    // FP64 for the predicted candidates beside the FP32 form, then FP64 for
-    // the ones the FP32 form could not certify
+    // FP64 for the predicted candidates beside the FP32 form (small calls:
+    // after it), then FP64 for the ones the FP32 form could not certify
     RR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     if ((rc = prepass())) return rc;
-    if ((rc = launch64(plan, ctx->side64))) return rc;
+    const bool beside = !join64 && !list64.empty();
+    if (beside && (rc = launch64(plan, ctx->side64))) return rc;
     if ((rc = fp32_run())) return rc;
-    if (!list64.empty()) {
+    if (beside) {
       RR_HIP(hipEventRecord(ctx->join64, ctx->side64));
       RR_HIP(hipStreamWaitEvent(ctx->stream, ctx->join64, 0));
     }
@@ -1863,12 +1875,13 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
     RR_HIP(hipStreamSynchronize(ctx->stream));
     std::vector<int32_t> again;
     for (int32_t c : list32) if (f32[c].flags & RR_F_NEEDS64) again.push_back(c);
+    if (join64) again.insert(again.end(), list64.begin(), list64.end());
     if (!again.empty()) {
       if ((rc = plan64(&again, 1, plan))) return rc;
       if ((rc = launch64(plan, ctx->stream))) return rc;
     }
-    rescored = list64;
-    rescored.insert(rescored.end(), again.begin(), again.end());
+    rescored.swap(again);
+    if (!join64) rescored.insert(rescored.end(), list64.begin(), list64.end());
   }
   if (!graph) RR_HIP(hipEventRecord(ev1, ctx->stream));
 

@@ -198,3 +198,25 @@ def test_fp32_streams_same_bits(ctx, count):
         assert got[0] == got[1] == got[2]
     ctx.set_option("fp32_streams", keep)
     ctx.free(h)
+
+
+@pytest.mark.parametrize("n", [9000, 20000])
+def test_checked_form_fp64_results_either_way(ctx, n):
+    """The candidates a checked call gives to FP64 take FP64's bits, scored
+    with the re-scores (few FP32 chunks) or beside the FP32 kernels."""
+    print("case: checked form n=%d" % n, flush=True)
+    import rils_rols_cpp
+    rng = np.random.default_rng(23)
+    X = rng.uniform(-5, 5, (n, 4))
+    y = np.sin(X[:, 0]) * X[:, 1] + rng.normal(0, 0.01, n)
+    facs = [rils_rols_cpp._ols_factors(t) for t in treegen.random_trees(23, 320, 3, 40, 4)]
+    arrs = capi.build_batch(facs)
+    h = ctx.upload(X, y)
+    c64, f64 = ctx.fitness(h, arrs, precision="fp64")
+    cc, fc = ctx.fitness(h, arrs, precision="fp32c")
+    ctx.free(h)
+    took = [i for i in range(len(facs)) if fc[i]["flags"] & capi.D["RR_F_FP64"]]
+    assert len(took) > 20
+    for i in took:
+        assert np.asarray(cc[i]).tobytes() == np.asarray(c64[i]).tobytes(), i
+        assert (fc[i]["e0"], fc[i]["e1"]) == (f64[i]["e0"], f64[i]["e1"]), i
