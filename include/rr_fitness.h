@@ -301,7 +301,7 @@ int rr_last_kernel_ms(rr_ctx* ctx, double* ms);
 #define RR_PHASE_PREPASS 0  /* k_nan0_fp64: factor 0 on the first 64 samples */
 #define RR_PHASE_EVAL 1     /* k_alive_fp64 + k_eval_fp64: the FP64 factor columns */
 #define RR_PHASE_QR 2       /* k_ts_* / k_qr_*: the column-pivoted QR and the solve */
-#define RR_PHASE_SCORE 3    /* k_score_fp64 + k_fit_fp64: prediction, SSR, R2, RMSE */
+#define RR_PHASE_SCORE 3    /* k_score_ols or k_score_raw, k_fit_fp64: prediction, SSR, R2, RMSE */
 #define RR_PHASE_FP32 4     /* the FP32 form's kernels (k_acc_fp32 + k_fin_fp32, or the raw pair) */
 /* host wall-clock parts of the last rr_fitness_* call (recorded whatever
  * "phase_timing" is): */

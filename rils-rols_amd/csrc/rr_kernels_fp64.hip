@@ -31,7 +31,7 @@
 //                 the same factorisation step by step over the columns in
 //                 HBM, every candidate of the launch in lockstep (described
 //                 below);
-//   k_score_fp64 + k_fit_fp64
+//   k_score_ols (k_score_raw) + k_fit_fp64
 //                 per (candidate, chunk) the OLS tree's prediction from the
 //                 coefficients and the kept columns (rils_rols_cpp.cpp:
 //                 488-517: left-deep sum of c*f, or f when |c-1| < 1e-12,
@@ -846,7 +846,7 @@ __device__ inline void qr_solve_pos(const QrArgs& a, int pos) {
     write_fit(a.fit + c.cand, rrm::qnan(), c.D->sst, c.n, r, s.steps);
     a.info[c.cand] = -1;
   } else {
-    a.info[c.cand] = r | (s.steps << 16);   // scored by k_score_fp64 / k_fit_fp64
+    a.info[c.cand] = r | (s.steps << 16);   // scored by k_score_ols / k_fit_fp64
   }
 }
 #undef NU
@@ -2297,7 +2297,7 @@ __global__ __launch_bounds__(WAVE) void k_ts_solve(TsArgs a) {
     write_fit(a.fit + cand, rrm::qnan(), D.sst, n, r, steps);
     a.info[cand] = -1;
   } else {
-    a.info[cand] = r | (steps << 16);   // scored by k_score_fp64 / k_fit_fp64
+    a.info[cand] = r | (steps << 16);   // scored by k_score_ols / k_fit_fp64
   }
 }
 
