@@ -28,3 +28,22 @@ def ctx():
     c = capi.Context(0)
     yield c
     c.close()
+
+
+OPTIONS = ("slab_budget_mb", "fp64_eval_rows", "fp64_eval_form", "fp32_rows", "fp32_chunk_rows", "fp32_streams",
+           "host_threads", "phase_timing", "graph")
+
+
+@pytest.fixture(autouse=True)
+def _options_put_back(request):
+    """Every test that uses the shared context finds it at its default options
+    (four FP64 rows a thread, bucket streams by size), whatever the tests
+    before it set or put back."""
+    if "ctx" not in request.fixturenames:
+        yield
+        return
+    c = request.getfixturevalue("ctx")
+    keep = [(k, c.get_option(k)) for k in OPTIONS]
+    yield
+    for k, v in keep:
+        c.set_option(k, v)

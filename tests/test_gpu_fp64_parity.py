@@ -733,3 +733,32 @@ def test_deep_stacks_at_four_rows_bitexact(ctx, n, levels):
     for t, tu, c, f in zip(trees, tuned, coefs, fit):
         assert same_bits(c, tu["coefs"]), (t, c, tu["coefs"])
         assert same_bits([f["e0"], f["e1"]], [tu["fit"][0], tu["fit"][1]]), (t, f, tu["fit"])
+
+
+def test_shared_context_is_at_its_defaults(ctx):
+    """After the tests above, which set options, the shared context still has
+    a new context's options."""
+    import conftest
+    fresh = capi.Context(0)
+    want = {k: fresh.get_option(k) for k in conftest.OPTIONS}
+    fresh.close()
+    assert {k: ctx.get_option(k) for k in conftest.OPTIONS} == want
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4])
+@pytest.mark.parametrize("n", [150, 600, 4097, 9000])
+def test_small_raw_batches_at_every_row_count(ctx, n, rows):
+    """Raw calls with their inputs in the launch's argument and staged ones at
+    one, two and four rows a thread."""
+    print("case: small raw batches n=%d rows=%d" % (n, rows), flush=True)
+    X, y = make_data(97, n, 3)
+    od = O.Dataset(X, y)
+    trees = treegen.random_trees(98, 60, 1, 40, 3)
+    want = [od.score(t)[:2] for t in trees]
+    h = ctx.upload(X, y)
+    ctx.set_option("fp64_eval_rows", rows)
+    for count in (1, 5, 60):
+        _, fit = ctx.fitness(h, capi.build_batch([[t] for t in trees[:count]]), mode="raw")
+        for t, f, w in zip(trees, fit, want):
+            assert same_bits([f["e0"], f["e1"]], w), t
+    ctx.free(h)
