@@ -762,3 +762,60 @@ def test_small_raw_batches_at_every_row_count(ctx, n, rows):
         for t, f, w in zip(trees, fit, want):
             assert same_bits([f["e0"], f["e1"]], w), t
     ctx.free(h)
+
+
+def _comb_batch(progs):
+    """Raw trees `op v0 (op v1 (... vk))` in the order written (left operand
+    first), which takes a stack slot per operator: few instructions, many
+    slots.  progs: (operators, variables) pairs; returns the batch and the
+    trees in prefix form."""
+    code, starts, trees = [], [0], []
+    for ops, xs in progs:
+        for x in xs[:-1]:
+            code += [(x << 8) | capi.D["RR_OP_LDV"], capi.D["RR_OP_PUSH"]]
+        code.append((xs[-1] << 8) | capi.D["RR_OP_LDV"])
+        code += [capi.D["RR_OP_BIN"] + 8 * capi.BINARY[op] + capi.D["RR_M_S"] for op in reversed(ops)]
+        starts.append(len(code))
+        trees.append(" ".join("%s x%d" % p for p in zip(ops, xs)) + (" x%d" % xs[-1]))
+    arrs = {"cand_start": np.arange(len(progs) + 1, dtype=np.int32), "prog_start": np.array(starts, dtype=np.int32),
+            "code": np.array(code, dtype=np.uint32), "consts": np.zeros(1), "n_consts": 0, "n_cands": len(progs)}
+    return arrs, trees
+
+
+# one to three chunks of rows; row counts that take two and four rows a thread
+@pytest.mark.parametrize("form,rows", [(1, 4), (1, 2), (1, 1), (0, 4), (0, 1)])
+@pytest.mark.parametrize("n", [512, 513, 4097, 9001])
+def test_raw_deep_stacks_bitexact(ctx, n, form, rows):
+    """Raw trees of 1 to 8 stack slots (8 is the most a program may take): up
+    to 7 slots the operand stack of four rows a thread fits the LDS a launch
+    may ask for, at 8 the launch takes two rows.  In calls small enough for the
+    launch's argument and staged ones, over two datasets, pipelined and without
+    allocation."""
+    print("case: raw deep stacks n=%d form=%d rows=%d" % (n, form, rows), flush=True)
+    assert capi.D["RR_MAX_STACK"] == 8
+    rng = np.random.default_rng(n)
+    progs = [([str(o) for o in rng.choice(["+", "-", "*", "max", "min"], slots)],
+              [int(x) for x in rng.integers(0, 4, slots + 1)])
+             for slots in (3, 8, 1, 4, 7, 2, 5, 6, 8, 3)] * 10
+    data = [make_data(95, n, 4), make_data(96, 150, 4)]
+    ods = [O.Dataset(X, y) for X, y in data]
+    hs = [ctx.upload(X, y) for X, y in data]
+    ctx.set_option("fp64_eval_rows", rows)
+    ctx.set_option("fp64_eval_form", form)
+
+    def check(fit, trees, which):
+        for t, f, w in zip(trees, fit, which):
+            e0, e1, _ = ods[w].score(t)
+            assert same_bits([f["e0"], f["e1"]], [e0, e1]), (w, t)
+    seven = [p for p in progs if len(p[0]) < 8]
+    for part in (progs[:1], seven[:8], seven, progs[:2], progs[:10], progs):
+        arrs, trees = _comb_batch(part)
+        check(ctx.fitness(hs[0], arrs, mode="raw")[1], trees, [0] * len(part))
+        check(ctx.fitness_noalloc(hs[0], arrs, mode="raw")[1], trees, [0] * len(part))
+        which = [i % 2 for i in range(len(part))]
+        check(ctx.fitness(None, arrs, mode="raw", handles=[hs[w] for w in which])[1], trees, which)
+        pending = ctx.submit(hs[0], arrs, mode="raw")
+        ctx.wait()
+        check(pending()[1], trees, [0] * len(part))
+    for h in hs:
+        ctx.free(h)
