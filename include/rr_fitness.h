@@ -288,8 +288,10 @@ int rr_autotune(rr_ctx* ctx, int32_t handle, const rr_batch* batch, int32_t mode
                 double* best_ms);
 int rr_get_option(rr_ctx* ctx, const char* name, int64_t* value);
 
-/* Kernel time of the last rr_fitness_batch / rr_predict call on the context's
- * stream, in milliseconds (HIP events around the launches). */
+/* Kernel time of the last rr_fitness_* / rr_predict / rr_predict_fp32 call on
+ * the context's stream, in milliseconds (HIP events around the launches); 0
+ * after rr_predict_rows, whose kernels run between the copies of its rows and
+ * are not timed. */
 int rr_last_kernel_ms(rr_ctx* ctx, double* ms);
 
 /* The same split by phase (HIP events around each phase's launches on the

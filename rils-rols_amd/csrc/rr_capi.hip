@@ -2110,6 +2110,7 @@ int rr_predict_rows(rr_ctx* ctx, const double* X_rm, int64_t n, int32_t d, const
                                    cnt(i), 1, d, (double*)ho(i), ctx->stream));
     RR_HIP(hipEventRecord(ctx->pdone[i % slots], ctx->stream));
   }
+  ctx->last_ms = 0.0;   // not timed, and no older call's time
   return RR_OK;
 }
 

@@ -65,6 +65,20 @@ def test_predict_rows_bitexact(ctx, n, d):
     assert same_bits(ctx.predict_rows(X, pre), O.Dataset(X, np.zeros(n)).eval(pre))
 
 
+def test_predict_rows_leaves_no_older_kernel_time(ctx):
+    """rr_last_kernel_ms after rr_predict_rows is 0, not an older call's time,
+    and the other entry points' own again after that."""
+    X, y = make_data(6, 3000, 2)
+    h = ctx.upload(X, y)
+    ctx.fitness(h, capi.build_batch([["sin x0"]]))
+    assert ctx.kernel_ms() > 0
+    ctx.predict_rows(X, "sin x0")
+    assert ctx.kernel_ms() == 0.0
+    ctx.predict(h, "sin x0", 3000)
+    assert ctx.kernel_ms() > 0
+    ctx.free(h)
+
+
 def test_predict_rows_argument_errors(ctx):
     for X, pre in [(np.zeros((0, 2)), "x0"), (np.zeros((4, 2)), "x2")]:
         with pytest.raises(RuntimeError):
