@@ -342,9 +342,8 @@ class BatchRunner {
     prog64_.assign(1, 0); code64_.clear(); consts64_.clear();
   }
   void add(const Flat& f) {
-    rrh::compile(f, code_, consts_);
+    rrh::compile_both(f, code_, consts_, code64_, consts64_, folder_);
     prog_.push_back((int32_t)code_.size());
-    rrh::compile_folded(f, code64_, consts64_, folder_);
     prog64_.push_back((int32_t)code64_.size());
   }
   // the prepared batch: constants folded for the FP64 form
@@ -516,6 +515,18 @@ PYBIND11_MODULE(rils_rols_cpp, m) {
   m.def("_fold", [](const std::string& prefix) {
     rrh::Folder folder;
     return rrh::to_prefix(folder.fold(rrh::parse_prefix(prefix)));
+  });
+  m.def("_compile_both", [](const std::vector<std::string>& prefixes) {
+    std::vector<uint32_t> code, code64;
+    std::vector<double> consts, consts64;
+    std::vector<size_t> ends, ends64;
+    rrh::Folder folder;
+    for (const std::string& p : prefixes) {
+      rrh::compile_both(rrh::parse_prefix(p), code, consts, code64, consts64, folder);
+      ends.push_back(code.size());
+      ends64.push_back(code64.size());
+    }
+    return py::make_tuple(py::make_tuple(code, consts, ends), py::make_tuple(code64, consts64, ends64));
   });
   m.def("_ols_tree", &ols_tree_hook);
   m.def("_crand", &rand_hook);

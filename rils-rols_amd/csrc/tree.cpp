@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <stdexcept>
+#include <string_view>
 
 #include "../../include/rr_fitness.h"
 
@@ -20,11 +21,10 @@ static const double EPS = 1e-12;   // node.h:13-14, pow(10, -12)
 static inline bool value_zero(double v) { return std::fabs(v) < EPS; }   // node.h:333-335
 static inline bool value_one(double v) { return std::fabs(v - 1) < EPS; } // node.h:337-339
 
-void subtree_sizes(const Flat& f, std::vector<int32_t>& size) {
+static void subtree_sizes(const Flat& f, std::vector<int32_t>& size, std::vector<int32_t>& st) {
   const int m = (int)f.size();
   size.resize(m);
-  std::vector<int32_t> st;
-  st.reserve(64);
+  st.clear();
   for (int i = m - 1; i >= 0; --i) {
     int32_t s = 1;
     for (int a = arity(f[i].t); a > 0; --a) {
@@ -36,6 +36,11 @@ void subtree_sizes(const Flat& f, std::vector<int32_t>& size) {
     st.push_back(s);
   }
   if (st.size() != 1) throw std::runtime_error("malformed prefix tree");
+}
+void subtree_sizes(const Flat& f, std::vector<int32_t>& size) {
+  std::vector<int32_t> st;
+  st.reserve(64);
+  subtree_sizes(f, size, st);
 }
 
 // std::to_string(int) / std::to_string(double) as used by node::to_string;
@@ -124,24 +129,28 @@ std::string to_prefix(const Flat& f) {
 
 Flat parse_prefix(const std::string& s) {
   Flat f;
+  f.reserve(32);
   size_t p = 0;
   while (p < s.size()) {
     while (p < s.size() && s[p] == ' ') ++p;
     size_t q = p;
     while (q < s.size() && s[q] != ' ') ++q;
     if (q == p) break;
-    const std::string t = s.substr(p, q - p);
+    const std::string_view t(s.data() + p, q - p);   // a number ends with its token: at a space or the string's end
     p = q;
-    if (t.size() > 1 && t[0] == 'c' && t != "cos") { f.push_back(tok_const(strtod(t.c_str() + 1, nullptr))); continue; }
-    if (t.size() > 1 && t[0] == 'x') { f.push_back(tok_var(atoi(t.c_str() + 1))); continue; }
+    if (t.size() > 1 && t[0] == 'c' && t != "cos") { f.push_back(tok_const(strtod(t.data() + 1, nullptr))); continue; }
+    if (t.size() > 1 && t[0] == 'x') { f.push_back(tok_var(atoi(t.data() + 1))); continue; }
     uint8_t ty = NONE;
-    for (uint8_t k = PLUS; k <= MAX; ++k) if (t == tok_name(k)) { ty = k; break; }
-    if (ty == NONE) throw std::runtime_error("bad prefix token: " + t);
+    for (uint8_t k = PLUS; k <= MAX; ++k) if (t[0] == *tok_name(k) && t == tok_name(k)) { ty = k; break; }
+    if (ty == NONE) throw std::runtime_error("bad prefix token: " + std::string(t));
     f.push_back(tok_op(ty));
   }
-  std::vector<int32_t> sz;
-  subtree_sizes(f, sz);
-  if (f.empty() || sz[0] != (int)f.size()) throw std::runtime_error("malformed prefix tree");
+  int64_t open = 1;   // operands still to come
+  for (size_t i = 0; i < f.size(); ++i) {
+    if (open == 0) throw std::runtime_error("malformed prefix tree");
+    open += arity(f[i].t) - 1;
+  }
+  if (open != 0) throw std::runtime_error("malformed prefix tree");
   return f;
 }
 
@@ -492,7 +501,7 @@ namespace {
 struct Emitter {
   const Flat& f;
   const std::vector<int32_t>& sz;
-  std::vector<int32_t> need;
+  std::vector<int32_t>& need;
   std::vector<uint32_t>& code;
   std::vector<double>& consts;
   int sp = 0, depth = 0;
@@ -563,15 +572,34 @@ void compile_folded(const Flat& f, std::vector<uint32_t>& code, std::vector<doub
     // what compile() refuses is refused here
     std::vector<uint32_t> c;
     std::vector<double> k;
-    compile(f, c, k);
+    compile(f, c, k, folder.work);
   }
-  compile(g, code, consts);
+  compile(g, code, consts, folder.work);
+}
+
+void compile_both(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts,
+                  std::vector<uint32_t>& code64, std::vector<double>& consts64, Folder& folder) {
+  const size_t c0 = code.size(), k0 = consts.size();
+  compile(f, code, consts, folder.work);
+  const Flat& g = folder.fold(f);
+  if (&g != &f) { compile(g, code64, consts64, folder.work); return; }
+  // nothing folded: the same instructions, constants by their places in the other pool
+  const uint32_t shift = (uint32_t)(consts64.size() - k0) << 8;
+  for (size_t i = c0; i < code.size(); ++i) {
+    const uint32_t op = code[i] & 0xffu, m = (op - RR_OP_BIN) & 7u;
+    const bool k = op >= RR_OP_BIN ? m == RR_M_C || m == RR_M_CR : op == RR_OP_LDC;
+    code64.push_back(k ? code[i] + shift : code[i]);
+  }
+  consts64.insert(consts64.end(), consts.begin() + (ptrdiff_t)k0, consts.end());
 }
 
 int compile(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts) {
-  std::vector<int32_t> sz;
-  subtree_sizes(f, sz);
-  Emitter e{f, sz, {}, code, consts};
+  CompileWork w;
+  return compile(f, code, consts, w);
+}
+int compile(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts, CompileWork& w) {
+  subtree_sizes(f, w.sz, w.st);
+  Emitter e{f, w.sz, w.need, code, consts};
   e.compute_need();
   e.gen(0);
   if (e.depth > RR_MAX_STACK) throw std::runtime_error("expression needs more operand-stack slots than RR_MAX_STACK");

@@ -102,10 +102,12 @@ struct Program {
 // carry out in every row (rr_math.h gives the same bits on the host), so the
 // program's values keep their bits.  Not for the FP32 form, whose bounds and
 // certificates are those of its own evaluation of the constants.
+struct CompileWork { std::vector<int32_t> sz, st, need; };   // compile's arrays, kept over programs
 class Folder {
  public:
   // f itself when there is nothing to fold, else a tree valid until the next call
   const Flat& fold(const Flat& f);
+  CompileWork work;
  private:
   struct Ent { bool cst; double v; size_t start; };   // a subtree: its tokens in rev_ begin at start
   Flat rev_, out_;
@@ -115,7 +117,12 @@ class Folder {
 // Appends the program of subtree `f` to `code`, its constants to `consts`.
 // Returns the operand-stack depth it needs.
 int compile(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts);
+int compile(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts, CompileWork& w);
 // The same for the FP64 form: the program of the folded tree.
 void compile_folded(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts, Folder& folder);
+// Both, for a batch that either form may score: compile to code / consts,
+// compile_folded to code64 / consts64.
+void compile_both(const Flat& f, std::vector<uint32_t>& code, std::vector<double>& consts,
+                  std::vector<uint32_t>& code64, std::vector<double>& consts64, Folder& folder);
 
 }  // namespace rrh

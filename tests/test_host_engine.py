@@ -14,6 +14,7 @@ import oracle_lib as O
 import treegen
 
 rrc = pytest.importorskip("rils_rols_cpp")
+D = capi.D
 
 
 def corpus(seed, count, lo, hi, nvars, ops=treegen.OPS):
@@ -111,6 +112,42 @@ def test_folded_constants_keep_the_values():
         assert np.all((u.view(np.uint64) == v.view(np.uint64)) | (np.isnan(u) & np.isnan(v))), (t, g)
     assert rrc._fold("+ x0 * x1 c0x1p+1") == "+ x0 * x1 c0x1p+1"
     assert rrc._fold("sin + c0x1p+0 c0x1p+1").startswith("c")
+
+
+def test_both_program_lists_are_those_of_each_tree():
+    """A prepared batch's two program lists: the compiled trees and the
+    compiled folded trees, each instruction with its own pool's constant."""
+    trees = treegen.random_trees(41, 400, 1, 40, 4) + treegen.random_trees(42, 200, 1, 30, 4, const_p=0.1)
+    trees += ["x3", "c0x1p+1", "+ x0 c0x1p+1", "- c0x1p+1 x0", "sin c0x1p+0", "* sin x0 cos / c0x1p+0 c0x0p+0",
+              "max c0x1p+2 x1", "< x0 c-0x0p+0"]
+
+    def decoded(code, consts):
+        out = []
+        for w in code:
+            op, arg = w & 0xff, w >> 8
+            k = op == D["RR_OP_LDC"] or op >= D["RR_OP_BIN"] and \
+                (op - D["RR_OP_BIN"]) % 8 in (D["RR_M_C"], D["RR_M_CR"])
+            out.append((op, np.float64(consts[arg]).tobytes() if k else arg))
+        return out
+    plain, folded = rrc._compile_both(trees)
+    kept = 0
+    for (code, consts, ends), prefix in ((plain, trees), (folded, [rrc._fold(t) for t in trees])):
+        assert len(ends) == len(trees) and ends[-1] == len(code)
+        for i, t in enumerate(prefix):
+            want, pool, _ = rrc._compile(t)
+            assert decoded(code[ends[i - 1] if i else 0:ends[i]], consts) == decoded(want, pool), t
+            kept += t == trees[i]
+    assert len(trees) < kept < 2 * len(trees)   # some folded, some not
+    with pytest.raises(Exception):   # too deep as written, whatever folds
+        def bal(d):
+            return "sin c0x1p+0" if d == 0 else "+ " + bal(d - 1) + " " + bal(d - 1)
+        rrc._compile_both([bal(9)])
+
+
+@pytest.mark.parametrize("bad", ["", " ", "+", "+ x0", "x0 x1", "sin", "+ x0 x1 x2", "foo", "c", "x", "cos", "+ x0 tan"])
+def test_malformed_prefix_trees_are_refused(bad):
+    with pytest.raises(RuntimeError):
+        rrc._compile(bad)
 
 
 def test_stack_depth_is_logarithmic():
