@@ -2365,7 +2365,7 @@ hipError_t launch_qr_solve(const QrLaunch& L, hipStream_t s) {
 constexpr size_t eval_stack(int depth, int rows) {
   return (size_t)(depth > 0 ? depth : 1) * (size_t)rows * EV_THREADS * sizeof(double);
 }
-constexpr size_t EVAL_LDS_MAX = 65536;   // what a launch asks for at most, static and dynamic
+constexpr size_t EVAL_LDS_MAX = 160 * 1024;   // what a gfx950 workgroup may ask for, static and dynamic
 
 hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s) {
   if (L.n_items <= 0) return hipSuccess;
@@ -2374,7 +2374,6 @@ hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s) {
   const dim3 grid((unsigned)L.n_items), block(EV_THREADS);
   // four rows: at most EVAL_LDS_SLOTS slots of four, which are enough for one row of any depth
   static_assert(4 * EVAL_LDS_SLOTS >= RR_MAX_STACK, "the stack of one row of a deep program");
-  static_assert(eval_stack(RR_MAX_STACK, 2) <= EVAL_LDS_MAX / 2, "the stack of two rows of any program");
   const size_t stk = eval_stack(L.rows == 4 ? std::min(L.depth, EVAL_LDS_SLOTS) : L.depth, L.rows);
   if (L.form == 1) {
     if (L.rows == 1) hipLaunchKernelGGL((k_eval_fp64<1, 1>), grid, block, stk, s, a);
@@ -2422,15 +2421,15 @@ hipError_t launch_nan0_fp64(const Nan0Launch& L, hipStream_t s) {
 }
 
 // the RAW kernel of the launch's rows and form
-#define RR_RAW_FORMS                       \
-  if (L.form == 1) {                       \
-    if (rows == 1) RR_RAW(1, 1, stk);      \
-    else if (rows == 4) RR_RAW(4, 1, stk); \
-    else RR_RAW(2, 1, stk);                \
-  } else {                                 \
-    if (rows == 1) RR_RAW(1, 0, 0);        \
-    else if (rows == 4) RR_RAW(4, 0, 0);   \
-    else RR_RAW(2, 0, 0);                  \
+#define RR_RAW_FORMS                         \
+  if (L.form == 1) {                         \
+    if (L.rows == 1) RR_RAW(1, 1, stk);      \
+    else if (L.rows == 4) RR_RAW(4, 1, stk); \
+    else RR_RAW(2, 1, stk);                  \
+  } else {                                   \
+    if (L.rows == 1) RR_RAW(1, 0, 0);        \
+    else if (L.rows == 4) RR_RAW(4, 0, 0);   \
+    else RR_RAW(2, 0, 0);                    \
   }
 hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {
   if (L.n_pos <= 0) return hipSuccess;
@@ -2445,16 +2444,16 @@ hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {
   const dim3 block(EV_THREADS), fgrid((unsigned)((L.n_pos + POS_THREADS - 1) / POS_THREADS));
   if (L.raw) {
     const dim3 grid((unsigned)L.n_items);
-    // Four rows a thread while the stack of the call's deepest tree and `red`
-    // fit EVAL_LDS_MAX (up to seven slots), else two.  900 trees on 50021 rows
-    // with one of 5, 6, 7, 8 slots among them (314 us of kernels without): four
-    // rows 484, 489, 828 us, two rows 549, 717, 1211, 2135 us; four rows, with
-    // trees of more than three slots one row at a time, 551, 940, 1745, 3322 us,
-    // and 352 us without one (the kernel then holds the interpreter twice).
-    constexpr size_t RED = EV_THREADS / WAVE * sizeof(double);
-    static_assert(eval_stack(RR_MAX_STACK - 1, 4) + RED <= EVAL_LDS_MAX, "seven slots of four rows");
-    const int rows = L.form == 1 && L.rows == 4 && eval_stack(L.depth, 4) + RED > EVAL_LDS_MAX ? 2 : L.rows;
-    const size_t stk = eval_stack(L.depth, rows);
+    // Sized for the call's deepest tree, 64 KiB at most (eight slots of four
+    // rows).  900 trees on 50021 rows take 314 us of kernels at three slots,
+    // and with one tree of 4, 5, 6, 7, 8 slots among them 391, 483, 489, 828,
+    // 1361 us; at two rows 546, 549, 717, 1211, 2228 us; with trees of more than
+    // three slots one row at a time, as k_eval_fp64 takes them, 356, 551, 940,
+    // 1745, 3322 us, and 352 us with none (the kernel then holds the interpreter
+    // twice).
+    static_assert(eval_stack(RR_MAX_STACK, 4) + EV_THREADS / WAVE * sizeof(double) <= EVAL_LDS_MAX,
+                  "the stack of the deepest tree and k_score_raw's sums");
+    const size_t stk = eval_stack(L.depth, L.rows);
     if (L.pack) {
       const ScorePackArgs pa{a, *L.pack};
 #define RR_RAW(R, F, STK) hipLaunchKernelGGL((k_score_raw_pack<R, F>), grid, block, STK, s, pa)

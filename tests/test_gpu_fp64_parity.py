@@ -800,11 +800,10 @@ def _comb_batch(progs):
 @pytest.mark.parametrize("form,rows", [(1, 4), (1, 2), (1, 1), (0, 4), (0, 1)])
 @pytest.mark.parametrize("n", [512, 513, 4097, 9001])
 def test_raw_deep_stacks_bitexact(ctx, n, form, rows):
-    """Raw trees of 1 to 8 stack slots (8 is the most a program may take): up
-    to 7 slots the operand stack of four rows a thread fits the LDS a launch
-    may ask for, at 8 the launch takes two rows.  In calls small enough for the
-    launch's argument and staged ones, over two datasets, pipelined and without
-    allocation."""
+    """Raw trees of 1 to 8 stack slots (8 is the most a program may take; form
+    1's LDS is sized by the call's deepest tree, up to 64 KiB), in calls small
+    enough for the launch's argument and staged ones, over two datasets,
+    pipelined and without allocation."""
     print("case: raw deep stacks n=%d form=%d rows=%d" % (n, form, rows), flush=True)
     assert capi.D["RR_MAX_STACK"] == 8
     rng = np.random.default_rng(n)
