@@ -256,9 +256,11 @@ int rr_predict_fp32(rr_ctx* ctx, int32_t handle, const uint32_t* code, int32_t l
  * may use for its per-candidate work columns, default 32768),
  * "fp64_eval_rows" (samples per thread per pass of the FP64 evaluation of
  * factors and trees: 1, 2 or 4, and no more than one pass of 256 threads over
- * the largest dataset needs; default 4), "fp64_eval_form" (the FP64
- * factor interpreter: 0 operand stack in registers and transcendentals
- * called, 1 operand stack in LDS and transcendentals inlined; default 1), "fp32_rows" (the same for the FP32 kernels: 1 or 2; default 2),
+ * the largest dataset needs, nor than 2 with fp64_eval_form 0; default 4),
+ * "fp64_eval_form" (the FP64 interpreter of factors and trees: 0 operand stack
+ * in registers and transcendentals called, 1 operand stack in LDS and
+ * transcendentals inlined; default 1), "fp32_rows" (samples per lane of the
+ * FP32 kernels: 1 or 2; default 2),
  * "fp32_chunk_rows" (samples per workgroup of the FP32 pass, a multiple of
  * 512; default 4096: a candidate's samples are split into chunks that run as
  * independent workgroups, and the chunk sums are added in chunk order),
@@ -276,9 +278,8 @@ int rr_predict_fp32(rr_ctx* ctx, int32_t handle, const uint32_t* code, int32_t l
 int rr_set_option(rr_ctx* ctx, const char* name, int64_t value);
 
 /* Autotuner: time `batch` (mode, precision) under every schedule of that
- * precision -- FP64: samples per thread of the evaluation 1, 2, 4 x
- * fp64_eval_form 0, 1; FP32:
- * samples per
+ * precision -- FP64: samples per thread of the evaluation 1, 2 x
+ * fp64_eval_form 0, 1, and 4 with form 1; FP32: samples per
  * lane 1, 2 x chunk rows 2048..16384 x bucket streams off/on -- taking the
  * best of `reps` runs each, and keep the fastest as the context's options
  * (read them back with rr_get_option).  FP64 results are the same bits under

@@ -1083,10 +1083,14 @@ int fitness_impl(rr_ctx* ctx, int32_t handle, const int32_t* handles, const rr_b
   }
   // rows per thread of the FP64 interpreters: the option's, but no more than
   // one pass of the workgroup's 256 threads needs for the largest dataset
-  // (rows past a dataset's end are evaluated for nothing)
+  // (rows past a dataset's end are evaluated for nothing), and at most two for
+  // form 0, whose operand stacks of four rows do not fit the registers (58
+  // spilled; 900 raw trees on 50021 rows: 4257 us of kernels at four rows, 624
+  // at two, 936 at one; the 4096-tree batch on 1e5 rows 5727, 1603, 1798)
   int64_t max_n = 1;
   for (const rr::DsDesc& t : table) max_n = std::max(max_n, t.n);
-  const int erows = (int)std::min<int64_t>(ctx->fp64_eval_rows, max_n <= 256 ? 1 : max_n <= 512 ? 2 : 4);
+  const int erows = (int)std::min<int64_t>(ctx->fp64_eval_rows,
+                                           max_n <= 256 ? 1 : max_n <= 512 || ctx->fp64_eval_form == 0 ? 2 : 4);
   auto ds_of = [&](int32_t c) -> const Dataset& { return ctx->ds[uniq[handles ? cand_ds[c] : 0]]; };
 
   // Which candidates go to which form.  RR_FP32_CHECKED: candidates with a
@@ -2157,7 +2161,8 @@ int rr_autotune(rr_ctx* ctx, int32_t handle, const rr_batch* b, int32_t mode, in
   std::vector<Cfg> cfgs;
   if (precision == RR_FP64) {
     for (int64_t e : {1, 2, 4})
-      for (int64_t f : {0, 1}) cfgs.push_back({e, f, 0});
+      for (int64_t f : {0, 1})
+        if (e < 4 || f == 1) cfgs.push_back({e, f, 0});
   } else {
     for (int64_t r : {1, 2})
       for (int64_t ch : {2048, 4096, 8192, 16384})

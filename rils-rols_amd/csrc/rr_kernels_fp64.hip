@@ -2381,7 +2381,6 @@ hipError_t launch_eval_fp64(const EvalLaunch& L, hipStream_t s) {
     else hipLaunchKernelGGL((k_eval_fp64<2, 1>), grid, block, stk, s, a);
   } else {
     if (L.rows == 1) hipLaunchKernelGGL((k_eval_fp64<1, 0>), grid, block, 0, s, a);
-    else if (L.rows == 4) hipLaunchKernelGGL((k_eval_fp64<4, 0>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((k_eval_fp64<2, 0>), grid, block, 0, s, a);
   }
   return hipGetLastError();
@@ -2428,7 +2427,6 @@ hipError_t launch_nan0_fp64(const Nan0Launch& L, hipStream_t s) {
     else RR_RAW(2, 1, stk);                  \
   } else {                                   \
     if (L.rows == 1) RR_RAW(1, 0, 0);        \
-    else if (L.rows == 4) RR_RAW(4, 0, 0);   \
     else RR_RAW(2, 0, 0);                    \
   }
 hipError_t launch_score_fp64(const ScoreLaunch& L, hipStream_t s) {

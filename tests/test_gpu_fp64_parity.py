@@ -778,6 +778,30 @@ def test_small_raw_batches_at_every_row_count(ctx, n, rows):
     ctx.free(h)
 
 
+def test_register_stack_form_keeps_to_two_rows(ctx):
+    """fp64_eval_form 0 at the default four rows a thread runs at two, which
+    its registers hold: the time of two rows asked for (spilled, four rows
+    take three to seven times as long)."""
+    print("case: register stack form, raw and OLS, n=50021", flush=True)
+    X, y = make_data(99, 50021, 4)
+    trees = treegen.random_trees(100, 100, 10, 30, 4)
+    od = O.Dataset(X[:100], y[:100])
+    h = ctx.upload(X, y)
+    ctx.set_option("fp64_eval_form", 0)
+    for mode, arrs in (("raw", capi.build_batch([[t] for t in trees])),
+                       ("ols", capi.build_batch([od.tune(t)["factors"] for t in trees]))):
+        best = {}
+        for rows in (2, 4):
+            ctx.set_option("fp64_eval_rows", rows)
+            times = []
+            for _ in range(6):
+                ctx.fitness(h, arrs, mode=mode)
+                times.append(ctx.kernel_ms())
+            best[rows] = min(times)
+        assert best[4] < 2 * best[2], (mode, best)
+    ctx.free(h)
+
+
 def _comb_batch(progs):
     """Raw trees `op v0 (op v1 (... vk))` in the order written (left operand
     first), which takes a stack slot per operator: few instructions, many
