@@ -197,10 +197,8 @@ __device__ inline void eval_f32(const uint32_t* __restrict__ code, int len, cons
 #pragma unroll
   for (int r = 0; r < R; ++r) { acc[r] = {0.f, 0.f}; st[r] = 0; }
   int sp = 0;
-  uint32_t next = code[0];   // the next instruction's word is on its way while one executes (1% of a call)
   for (int pc = 0; pc < len; ++pc) {
-    const uint32_t ins = next;
-    next = code[pc + 1 < len ? pc + 1 : pc];
+    const uint32_t ins = code[pc];   // (the next word fetched ahead, as eval_lds_f64 does, costs 1 to 4% here)
     const uint32_t op = ins & 0xffu;
     const uint32_t arg = ins >> 8;
     if (op >= RR_OP_BIN) {
