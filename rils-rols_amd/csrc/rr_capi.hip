@@ -192,7 +192,7 @@ struct rr_ctx {
   int64_t graph_made = 0, graph_updated = 0;   // executable graphs instantiated / reused
   size_t up_lo = SIZE_MAX, up_hi = 0;   // the staged bytes not yet copied
   int64_t slab_budget_mb = 32768;
-  int64_t fp64_eval_rows = 4;    // rows per thread and pass, at most (eval_rows)
+  int64_t fp64_eval_rows = 4;    // rows per thread and pass, at most (fitness_impl's erows)
   int64_t fp64_eval_form = 1;    // the factor interpreter: 0 stack in registers, 1 stack in LDS
   int64_t fp32_rows = 2;
   int64_t fp32_chunk_rows = 4096;
@@ -244,8 +244,8 @@ int set_device(rr_ctx* ctx) {
 // A side stream, made at its first use: most contexts run the plain FP64 form
 // only, and a stream costs 0.4 ms to destroy (and milliseconds to create
 // where its hardware queue is new to the process).  A search of 8000 calls on
-// 20003 rows, context and all: 18.5 ms with the five side streams, 14.5
-// without.
+// 20003 rows, context and all: 18.9 and 20.7 ms (two runs) with the five side
+// streams made with the context, 17.5 and 19.7 without.
 int make_side(hipStream_t* s) {
   if (!*s) RR_HIP(hipStreamCreateWithFlags(s, hipStreamNonBlocking));
   return RR_OK;
@@ -786,9 +786,10 @@ int rr_dataset_upload(rr_ctx* ctx, const double* X_fm, const double* y, int64_t 
   D.ldx = (n + rr::RR_ROW_PAD - 1) / rr::RR_ROW_PAD * rr::RR_ROW_PAD;   // whole tiles, never read past a column
   // One allocation for the dataset, and its input [columns | y] through two
   // pinned slots, as one flat array: while the GPU copies and places one piece,
-  // the host fills the other slot.  (With five allocations and pageable copies
-  // of columns and y, and FP32 copy, norms and statistics one pass each: 30000 x
-  // 6 rows 215 us, UPA now; 1e6 x 5 rows 3.9 ms, UPB; 150 x 2 rows 110 us, UPC.)
+  // the host fills the other slot.  With five allocations and pageable copies
+  // of columns and y, and FP32 copy, norms and statistics one pass each: 150 x 2
+  // rows 99 us, 28 now; 30000 x 6 232, 116; 1e5 x 10 596, 366; 1e6 x 5 4.6 ms,
+  // 1.6.
   const size_t cols = (size_t)std::max(d, 1), lb = (size_t)D.ldx * sizeof(double);
   const size_t o_y = lb * cols, o_one = o_y + lb, o_x32 = o_one + lb, o_norm = o_x32 + lb / 2 * cols;
   const size_t chunks = (size_t)(D.ldx / rr::EVAL_CHUNK_ROWS);

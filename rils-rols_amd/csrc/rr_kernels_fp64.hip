@@ -958,7 +958,7 @@ __global__ __launch_bounds__(QR_THREADS) void k_qr_all1(QrArgs a) {
 // k_qr_all1 (thread 0 alone on the serial parts, five barriers, the columns in global
 // memory) 270 us.
 constexpr int QS_THREADS = 512;
-constexpr size_t QS_LDS = 60 * 1024;   // for the columns, of the 64 KiB a workgroup may ask for
+constexpr size_t QS_LDS = 60 * 1024;   // for the columns: two workgroups of eight waves per compute unit
 // 12 WAVE rows of more than TS_MAX_COLS + 1 columns with y exceed QS_LDS
 static_assert((TS_MAX_COLS + 2) * 12 * WAVE * sizeof(double) > QS_LDS, "rows that fit LDS fit k_qr_small's registers");
 template <int RG>
@@ -1201,9 +1201,9 @@ static_assert(EVAL_CHUNK_ROWS == rrm::NORM_CHUNK, "evaluation work items are the
 // raw trees on 50021 rows, of the 4096-tree batch on 1e5 rows: 919, 1816 us
 // at one row, 554, 1460 at two, 462, 1425 at four and five waves, 428, 1380
 // at four and six, 430, 1545 at eight rows and four waves.
-constexpr int eval_waves(int, int form) { return form == 0 ? 8 : 6; }
+constexpr int eval_waves(int form) { return form == 0 ? 8 : 6; }
 template <int R, int FORM>
-__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_eval_fp64(EvalArgs a) {
+__global__ __launch_bounds__(EV_THREADS, eval_waves(FORM)) void k_eval_fp64(EvalArgs a) {
   static_assert(EV_THREADS == rrm::NORM_PARTIALS, "one thread per partial of the chunked order");
   __shared__ double red[EV_THREADS / WAVE][2];
   extern __shared__ double ev_stk[];
@@ -1497,10 +1497,11 @@ __device__ inline void score_finish(const ScoreArgs& a, double s, double (&red)[
 
 // RAW: one workgroup per work item, the candidate's one program over the chunk.
 // FORM as in k_eval_fp64, whose interpreters and register budgets these are.
-// Bound by the interpreter's latencies and its instruction issue (58% busy): a
-// call of 900 trees of about 20 nodes on 50021 rows takes 475 us with the
-// operand stack in LDS and four rows a thread, 611 with two rows, and took 840
-// with the stack in registers and the transcendentals called.
+// Bound by the interpreter's latencies and its instruction issue (57% busy): 900
+// trees of about 20 nodes on 50021 rows take 428 us of kernels with the operand
+// stack in LDS and four rows a thread, 594 with two rows, 1024 with one, and
+// with the stack in registers and the transcendentals called 624 (two rows),
+// 936 (one).
 template <int R, int FORM>
 __device__ inline void score_raw(const ScoreArgs& a, double (&red)[EV_THREADS / WAVE], double* sc_stk) {
   const int item = (int)blockIdx.x;
@@ -1530,7 +1531,7 @@ __device__ inline void score_raw(const ScoreArgs& a, double (&red)[EV_THREADS / 
   score_finish(a, s, red, item, D, cand, 0);
 }
 template <int R, int FORM>
-__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_raw(ScoreArgs a) {
+__global__ __launch_bounds__(EV_THREADS, eval_waves(FORM)) void k_score_raw(ScoreArgs a) {
   __shared__ double red[EV_THREADS / WAVE];
   extern __shared__ double sc_stk[];   // FORM 1: the operand stack
   score_raw<R, FORM>(a, red, sc_stk);
@@ -1558,7 +1559,7 @@ __device__ inline ScoreArgs unpack_args() {
   return a;
 }
 template <int R, int FORM>
-__global__ __launch_bounds__(EV_THREADS, eval_waves(R, FORM)) void k_score_raw_pack(ScorePackArgs) {
+__global__ __launch_bounds__(EV_THREADS, eval_waves(FORM)) void k_score_raw_pack(ScorePackArgs) {
   __shared__ double red[EV_THREADS / WAVE];
   extern __shared__ double sc_stk[];   // FORM 1: the operand stack
   score_raw<R, FORM>(unpack_args(), red, sc_stk);

@@ -5,6 +5,10 @@ The GPU kernels and the oracle implement the same canonical arithmetic
 operation order), so coefficients, 1-R2 and RMSE must be identical bits; the
 only allowance is the sign of a NaN produced by a hardware operation (x86 and
 AMDGPU default NaNs differ), which is compared as "both NaN".
+
+Tests that set no option run at a new context's: form 1 at four rows a thread
+(two up to 512 rows, one up to 256).  Form 0 runs at two where four are asked
+for, and raw trees run the form asked for at every stack depth.
 """
 import numpy as np
 import pytest
